@@ -94,13 +94,21 @@ struct KParams {
 
 // ---------------------------------------------------------------- work distribution
 
-// Workgroups are dealt round-robin to the 8 XCDs (each with its own L2). Map consecutive logical
-// tiles onto one XCD so that neighbouring tiles share their source footprints in that L2.
+// Workgroups are dealt round-robin to the 8 XCDs (each with its own L2). Runs of XCD_RUN
+// consecutive logical tiles go to one XCD, so that neighbouring tiles share their source footprints
+// in that L2, and the runs are dealt to the XCDs in turn, so that every XCD gets its share of the
+// costly and of the cheap parts of each view. (One contiguous eighth of the tiles per XCD left
+// XCDs idle while the one with the costliest eighth finished: 1.7 of 2 wave slots per SIMD were
+// taken on average. 9 views of 1920 x 1080 with 6 sources: half step 24.9 -> 23.5 ms; 2 such
+// views from a random start: 38.8 -> 35.3 ms a run of 3 iterations. Runs of 4 and 8 tiles measured
+// 3 and 2 % slower in the half step, 64 and 256 1 % slower.) The tiles after the last whole round
+// keep their order.
+constexpr int XCD_RUN = 16;
 __device__ __forceinline__ int xcd_tile(int bid, int n) {
     const int nx = 8;
-    int q = n / nx, r = n % nx;
-    int x = bid % nx, k = bid / nx;
-    return x * q + (x < r ? x : r) + k;
+    if (bid >= n - n % (nx * XCD_RUN)) return bid;
+    const int x = bid % nx, k = bid / nx;
+    return (k / XCD_RUN * nx + x) * XCD_RUN + k % XCD_RUN;
 }
 
 // Finds the batch item of flattened tile `t` for tiles of tw x th pixels; returns the item and
