@@ -10,7 +10,7 @@ struct KernelSet {
     int wr, wstep;
     hipError_t (*half)(const KParams&, int rows, int tpp, hipStream_t);
     hipError_t (*eval)(const KParams&, int mode, hipStream_t);
-    // cost of the pixels of colour P.color only (P.ntiles = half_tiles(items, 4, 1)), no initialisation
+    // cost of the pixels of colour P.color only (P.ntiles = span_tiles(items)), no initialisation
     hipError_t (*eval_color)(const KParams&, hipStream_t);
     hipError_t (*filter)(const KParams&, hipStream_t);
     hipError_t (*pair_costs)(const KParams&, int view, int slot, int n, const int* xy, const float4* planes, float* out,
@@ -28,6 +28,7 @@ bool half_shape_ok(int rows, int tpp);
 
 // workgroup counts of the two tilings for a batch
 int half_tiles(const BatchItem* items, int n, int rows, int tpp);
+int span_tiles(const BatchItem* items, int n);
 int pix_tiles(const BatchItem* items, int n);
 
 hipError_t launch_sample_reciprocal(const float* z, float* r, long long n, hipStream_t s);

@@ -212,7 +212,7 @@ struct c3d_pm_session {
     std::vector<BatchItem> h_batch_lv;
     std::vector<long long> h_snap_lv;
     std::vector<uint8_t> h_need;
-    // half-step workgroup shape: rows of active pixels and lanes per pixel (options.tile_rows and
+    // half-step workgroup shape: rows of pixel blocks and lanes per pixel (options.tile_rows and
     // options.threads_per_pixel, or c3d_pm_autotune)
     int half_rows = 1;
     int half_tpp = 1;
@@ -395,7 +395,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
         HIP_TRY(launch_eval_init(k, npix, st));
         KParams e = k;
         e.color = 1;
-        e.ntiles = half_tiles(items.data(), (int)items.size(), 4, 1);
+        e.ntiles = span_tiles(items.data(), (int)items.size());
         HIP_TRY(launch_span_tile_prefix(e.batch, e.nitems, s->tile_pre.p, st));
         e.tile_pre = s->tile_pre.p;
         HIP_TRY(s->ks->eval_color(e, st));

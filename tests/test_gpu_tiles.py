@@ -1,0 +1,43 @@
+"""Sizes at the edges of the half step's pixel blocks (16 x 8 pixels a wave with one lane per pixel)
+and of the runs of 16 tiles that are dealt to the 8 XCDs (128 tiles a round): the engine equals the
+oracle bit for bit under every workgroup shape."""
+import numpy as np
+import pytest
+
+from cumulus3d_amd import abi, pm, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes", [
+    [(16, 8), (15, 7), (17, 9)],          # one block, one pixel less, one more
+    [(31, 33), (8, 64), (240, 8)],        # remainders in both directions, one block high
+    [(256, 64), (240, 64), (257, 64)],    # 128, 120 and 136 blocks: a whole round, under it, over it
+])
+def test_block_edges_bit_exact(sizes):
+    import oracle
+
+    sc = scenes.make_mixed_scene(scenes.oblique_rig(3), sizes, seed=21)
+    pmp, fl = abi.fast_profile()
+    inp = scenes.kernel_input(sc, [[1, 2], [0, 2], [0, 1]], [(15.0, 120.0)] * 3, pmp, fl)
+
+    def run(engine):
+        st = [abi.ViewState(w, h) for w, h in sizes]
+        engine.run([0, 1, 2], st, abi.run_params(0, False, True, 1, 1, False))
+        snap = abi.DepthSnapshot(5, 0, [x.depth.copy() for x in st])
+        engine.run([0, 1, 2], st, abi.run_params(0, True, False, 1, 2, False), snap)
+        return st, engine.filter([0, 1, 2], st, snap)
+
+    ref, rc = run(oracle.Oracle(inp, threads=16))
+    for rows, tpp in [(0, 0)] + list(abi.TILE_SHAPES):
+        opts = abi.c3d_pm_options()
+        opts.tile_rows, opts.threads_per_pixel = rows, tpp
+        be = pm.HipPatchMatch(0, opts)
+        with be.begin(inp) as s:
+            got, gc = run(s)
+        be.close()
+        for a, b in zip(got, ref):
+            for x, y in ((a.depth, b.depth), (a.normal, b.normal), (a.cost, b.cost)):
+                assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32)), (rows, tpp)
+        for a, b in zip(gc, rc):
+            assert np.array_equal(a, b), (rows, tpp)
