@@ -233,8 +233,9 @@ __device__ __forceinline__ void c3d_sincosf(float x, float& so, float& co) {
 // hardware estimate v_rcp_f32 plus one Newton step would be the correctly rounded quotient, but
 // v_rcp_f32 issues at a quarter of the rate and measured slower (26.65 against 27.21 ms per half
 // step on 7 x 1920x1080 with 6 sources).
+__device__ __forceinline__ float rcp_seed(float z) { return __uint_as_float(0x7EF311C3u - __float_as_uint(z)); }
 __device__ __forceinline__ float rcp_sample(float z) {
-    float r = __uint_as_float(0x7EF311C3u - __float_as_uint(z));
+    float r = rcp_seed(z);
     float e = fmaf(-z, r, 1.0f);
     r = fmaf(r, fmaf(e, e, e), r);
     e = fmaf(-z, r, 1.0f);
@@ -299,6 +300,12 @@ struct RefTile {
     int x0, y0;
     __device__ __forceinline__ float at(int x, int y) const { return s[(y - y0) * TW + (x - x0)]; }
 };
+
+__device__ __forceinline__ float bilateral_weight(const KParams& P, float ic, float v, int dx, int dy) {
+    float d = ic - v;
+    float sp = (float)(dx * dx + dy * dy) * P.inv2s;
+    return c3d_expf(-fmaf(d * d, P.inv2c255, sp));
+}
 
 template <int WR, int WSTEP, class REF>
 __device__ __forceinline__ void ref_stats(const KParams& P, const REF& ref, int x, int y, RefWin<WR, WSTEP>& rw) {
@@ -372,10 +379,10 @@ __device__ __forceinline__ bool homography(const LevelDesc& R, const LevelPair& 
 // integers of magnitude below 2^11 and so exact. Each row is then one mixed FMA on the exact
 // half-float operands: the same value as the FP32 formula, in 8 instructions instead of 10.
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t quad_lo(uint32_t q) { return __builtin_amdgcn_perm(0x64646464u, q, 0x04020400u); }  // (1024 + p00, 1024 + p01)
+__device__ __forceinline__ uint32_t quad_hi(uint32_t q) { return __builtin_amdgcn_perm(0x64646464u, q, 0x04030401u); }  // (1024 + p10, 1024 + p11)
 __device__ __forceinline__ float quad_lerp(uint32_t q, float ax, float ay) {
-    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, q, 0x04020400u);  // (1024 + p00, 1024 + p01)
-    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, q, 0x04030401u);  // (1024 + p10, 1024 + p11)
-    const half2_t l = __builtin_bit_cast(half2_t, lo), h = __builtin_bit_cast(half2_t, hi);
+    const half2_t l = __builtin_bit_cast(half2_t, quad_lo(q)), h = __builtin_bit_cast(half2_t, quad_hi(q));
     const half2_t d = h - l;
     const half2_t p = l - (half2_t){(_Float16)1024.0f, (_Float16)1024.0f};
     const float top = fmaf(ax, (float)d.x, (float)p.x);
@@ -387,13 +394,18 @@ __device__ __forceinline__ float quad_lerp(uint32_t q, float ax, float ay) {
 // the table's first entry (x0, y0) = (-2, -2); the byte offset 4 ((y0 + 2) qpitch + (x0 + 2)) is formed
 // exactly in FP32 (multiples of 4 below 2^26) from the clamped floor of the sample position, and the
 // load uses a uniform base plus a 32-bit offset.
+__device__ __forceinline__ uint32_t quad_fetch(const uint32_t* qbase, float qp4, float koff4, float w1, float h1, float u, float v,
+                                               float& ax, float& ay) {
+    const float xf = floorf(u), yf = floorf(v);
+    ax = u - xf;
+    ay = v - yf;
+    const float xc = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
+    const float yc = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
+    return *(const uint32_t*)((const char*)qbase + (uint32_t)fmaf(yc, qp4, fmaf(xc, 4.0f, koff4)));
+}
 __device__ __forceinline__ float quad_sample(const uint32_t* qbase, float qp4, float koff4, float w1, float h1, float u, float v) {
-    float xf = floorf(u), yf = floorf(v);
-    float ax = u - xf, ay = v - yf;
-    float xc = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
-    float yc = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
-    uint32_t off = (uint32_t)fmaf(yc, qp4, fmaf(xc, 4.0f, koff4));
-    uint32_t q = *(const uint32_t*)((const char*)qbase + off);
+    float ax, ay;
+    const uint32_t q = quad_fetch(qbase, qp4, koff4, w1, h1, u, v, ax, ay);
     return quad_lerp(q, ax, ay);
 }
 
@@ -418,52 +430,139 @@ template <int WR, int WSTEP, bool CHECK, int PIPE, bool AHEAD, class REF>
 __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y, const uint32_t* qbase, float qp4,
                                             float koff4, float w1, float h1, const float* H, float& Ss, float& SSs, float& IS) {
     constexpr int WN = Win<WR, WSTEP>::WN;
+    constexpr int N = WN * WN;
     Ss = 0.f;
     SSs = 0.f;
     IS = 0.f;
-    // A rolling pipeline over the row-major samples: the gather of sample k + PIPE is issued
-    // before sample k is consumed, so PIPE gathers stay in flight. The sums take the samples in
-    // row-major order as before.
-    constexpr int N = WN * WN;
+    // A rolling pipeline over the row-major samples: the gather of sample k + PIPE is issued before
+    // sample k is used up, so PIPE gathers stay in flight. The sums take the samples in row-major
+    // order.
     float fx[N], fy[N], rv[N];
     uint32_t qv[N];
+    float rz = 0.f, ru = 0.f, rt = 0.f;  // the issued row's projective terms at dx = 0
+    auto xoff = [](int k) { return -WR + (k % WN) * WSTEP; };
+    auto yoff = [](int k) { return -WR + (k / WN) * WSTEP; };
+    auto row = [&](int k) {
+        const float oy = (float)yoff(k);
+        rz = fmaf(H[7], oy, H[8]);
+        ru = fmaf(H[1], oy, H[2]);
+        rt = fmaf(H[4], oy, H[5]);
+    };
     auto issue = [&](int k) {
-        const int a = k / WN, b = k % WN;
-        if constexpr (AHEAD) rv[k] = ref.at(x + (-WR + b * WSTEP), y + (-WR + a * WSTEP));
-        const float oy = (float)(-WR + a * WSTEP);
-        const float ox = (float)(-WR + b * WSTEP);
-        const float zz = fmaf(H[6], ox, fmaf(H[7], oy, H[8]));
-        const float r = rcp_sample(zz);
-        const float u = fmaf(H[0], ox, fmaf(H[1], oy, H[2])) * r, v = fmaf(H[3], ox, fmaf(H[4], oy, H[5])) * r;
-        const float xf = floorf(u), yf = floorf(v);
-        fx[k] = u - xf;
-        fy[k] = v - yf;
-        const float xc = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
-        const float yc = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
-        const uint32_t off = (uint32_t)fmaf(yc, qp4, fmaf(xc, 4.0f, koff4));
-        qv[k] = *(const uint32_t*)((const char*)qbase + off);
+        if (k % WN == 0) row(k);
+        if constexpr (AHEAD) rv[k] = ref.at(x + xoff(k), y + yoff(k));
+        const float ox = (float)xoff(k);
+        const float r = rcp_sample(fmaf(H[6], ox, rz));
+        qv[k] = quad_fetch(qbase, qp4, koff4, w1, h1, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rt) * r, fx[k], fy[k]);
     };
 #pragma unroll
     for (int k = 0; k < PIPE && k < N; ++k) issue(k);
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        if (k + PIPE < N) issue(k + PIPE);
-        const int a = k / WN, b = k % WN;
-        const uint32_t q = qv[k];
-        const float ax = fx[k], ay = fy[k];
-        float sv = quad_lerp(q, ax, ay);
-        if (CHECK) sv = fmaf(H[6], (float)(-WR + b * WSTEP), fmaf(H[7], (float)(-WR + a * WSTEP), H[8])) > 1e-8f ? sv : 0.0f;
-        float sp = sv - rw.ic;
-        float ws = rw.w[k] * sp;
+        // the operations of issue(n) and those on sample k in turn: written one after the other,
+        // the compiler needs more registers and spills at three waves per SIMD (half step 21.4
+        // instead of 20.0 ms on 9 views of 1920 x 1080); at two waves the order makes no difference
+        const int n = k + PIPE < N ? k + PIPE : N - 1;
+        const bool more = k + PIPE < N;
+        float zz, r, e, u, v, xf, yf;
+        if (more) {
+            if (n % WN == 0) row(n);
+            if constexpr (AHEAD) rv[n] = ref.at(x + xoff(n), y + yoff(n));
+            zz = fmaf(H[6], (float)xoff(n), rz);
+        }
+        const uint32_t lo = quad_lo(qv[k]);
+        if (more) r = rcp_seed(zz);
+        const uint32_t hi = quad_hi(qv[k]);
+        if (more) e = fmaf(-zz, r, 1.0f);
+        const half2_t l = __builtin_bit_cast(half2_t, lo);
+        const half2_t d = __builtin_bit_cast(half2_t, hi) - l;
+        if (more) e = fmaf(e, e, e);
+        const half2_t p = l - (half2_t){(_Float16)1024.0f, (_Float16)1024.0f};
+        if (more) r = fmaf(r, e, r);
+        const float top = fmaf(fx[k], (float)d.x, (float)p.x);
+        if (more) e = fmaf(-zz, r, 1.0f);
+        const float bot = fmaf(fx[k], (float)d.y, (float)p.y);
+        if (more) u = fmaf(H[0], (float)xoff(n), ru);
+        const float dv = bot - top;
+        if (more) r = fmaf(r, e, r);
+        float sv = fmaf(fy[k], dv, top);
+        if (CHECK) sv = fmaf(H[6], (float)xoff(k), fmaf(H[7], (float)yoff(k), H[8])) > 1e-8f ? sv : 0.0f;
+        if (more) v = fmaf(H[3], (float)xoff(n), rt);
+        const float sp = sv - rw.ic;
+        if (more) u = u * r;
+        const float ws = rw.w[k] * sp;
+        if (more) {
+            v = v * r;
+            xf = floorf(u);
+        }
         Ss += ws;
+        if (more) yf = floorf(v);
         SSs = fmaf(ws, sp, SSs);
-        IS = fmaf(ws, AHEAD ? rv[k] : ref.at(x + (-WR + b * WSTEP), y + (-WR + a * WSTEP)), IS);
+        if (more) fx[n] = u - xf;
+        IS = fmaf(ws, AHEAD ? rv[k] : ref.at(x + xoff(k), y + yoff(k)), IS);
+        if (more) {
+            xf = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
+            fy[n] = v - yf;
+            yf = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
+            xf = fmaf(xf, 4.0f, koff4);
+            qv[n] = *(const uint32_t*)((const char*)qbase + (uint32_t)fmaf(yf, qp4, xf));
+        }
+    }
+}
+
+// window_sums with CHECK as a loop over groups of CH samples that recomputes the bilateral weights;
+// same values and order. Windows that need the check are rare (0.4 to 2 % of a wave's windows have
+// such a lane, over runs on 1920 x 1080 and 960 x 540 views). A second unrolled copy of the window
+// beside the first one costs registers all the same (the compiler hoists what the two have in
+// common above the branch: 247 VGPRs instead of 192 in the photometric half step) and drains the
+// first gathers there. Groups of one sample measured 2 % slower on one 960 x 540 view, of six
+// 3 % slower on 9 views of 1920 x 1080 (spills).
+template <int WR, int WSTEP, class REF>
+__device__ __forceinline__ void window_sums_behind(const KParams& P, const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y,
+                                                   const uint32_t* qbase, float qp4, float koff4, float w1, float h1, const float* H,
+                                                   float& Ss, float& SSs, float& IS) {
+    constexpr int WN = Win<WR, WSTEP>::WN;
+    constexpr int CH = 3;
+    Ss = 0.f;
+    SSs = 0.f;
+    IS = 0.f;
+#pragma unroll 1
+    for (int a = 0; a < WN; ++a) {
+        const int dy = -WR + a * WSTEP;
+        const float oy = (float)dy;
+        const float rz = fmaf(H[7], oy, H[8]), ru = fmaf(H[1], oy, H[2]), rv = fmaf(H[4], oy, H[5]);
+#pragma unroll 1
+        for (int b0 = 0; b0 < WN; b0 += CH) {
+            float fx[CH], fy[CH], zs[CH];
+            uint32_t qv[CH];
+#pragma unroll
+            for (int g = 0; g < CH; ++g) {
+                const float ox = (float)(-WR + (b0 + g) * WSTEP);
+                zs[g] = fmaf(H[6], ox, rz);
+                const float r = rcp_sample(zs[g]);
+                qv[g] = quad_fetch(qbase, qp4, koff4, w1, h1, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r, fx[g], fy[g]);
+            }
+#pragma unroll
+            for (int g = 0; g < CH; ++g) {
+                if (WN % CH != 0 && b0 + g >= WN) break;
+                const int dx = -WR + (b0 + g) * WSTEP;
+                const float sv = zs[g] > 1e-8f ? quad_lerp(qv[g], fx[g], fy[g]) : 0.0f;
+                const float iv = ref.at(x + dx, y + dy);
+                const float sp = sv - rw.ic;
+                const float ws = bilateral_weight(P, rw.ic, iv, dx, dy) * sp;
+                Ss += ws;
+                SSs = fmaf(ws, sp, SSs);
+                IS = fmaf(ws, iv, IS);
+            }
+        }
     }
 }
 
 // Bilateral-weighted NCC cost 1 - rho, 2 on failure (patchmatch.cu:244-290); the covariance is
 // sum(w s' I)/W - mu mean(s') with s' the shifted source samples.
-template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool AHEAD = false, class REF>
+// COPY: windows with a sample behind the source take an unrolled copy of the window (short latency,
+// many registers) instead of the loop.
+template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool AHEAD = false, bool COPY = false, class REF>
 __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WSTEP>& rw, const REF& ref, const LevelDesc& S,
                                           const float* H, int x, int y) {
     float z = H[8];
@@ -481,8 +580,13 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
     const bool all_front = fmaf(H[6], lo, za) > 1e-8f && fmaf(H[6], hi, za) > 1e-8f && fmaf(H[6], lo, zb) > 1e-8f &&
                            fmaf(H[6], hi, zb) > 1e-8f;
     float Ss, SSs, IS;
-    if (all_front) window_sums<WR, WSTEP, false, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
-    else window_sums<WR, WSTEP, true, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+    if (all_front) {
+        window_sums<WR, WSTEP, false, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+    } else if constexpr (COPY) {
+        window_sums<WR, WSTEP, true, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+    } else {
+        window_sums_behind<WR, WSTEP>(P, rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+    }
     const float iW = rw.iW;
     float mus = Ss * iW;
     float vars = fmaf(-mus, mus, SSs * iW);
@@ -512,12 +616,6 @@ struct RefTileDyn {
 
 template <int WR, int WSTEP>
 using RefWinT = typename std::conditional<(WR > 0), RefWin<WR, WSTEP>, RefWinDyn>::type;
-
-__device__ __forceinline__ float bilateral_weight(const KParams& P, float ic, float v, int dx, int dy) {
-    float d = ic - v;
-    float sp = (float)(dx * dx + dy * dy) * P.inv2s;
-    return c3d_expf(-fmaf(d * d, P.inv2c255, sp));
-}
 
 template <int WSTEP, class REF>
 __device__ void ref_stats_dyn(const KParams& P, const REF& ref, int x, int y, int wr, RefWinDyn& rw) {
@@ -647,10 +745,10 @@ __device__ __forceinline__ void ref_stats_any(const KParams& P, const REF& ref, 
     else ref_stats_dyn<WSTEP>(P, ref, x, y, wr, rw);
 }
 
-template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool CHUNK = false, bool AHEAD = false, class REF>
+template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool CHUNK = false, bool AHEAD = false, bool COPY = false, class REF>
 __device__ __forceinline__ float ncc_cost_any(const KParams& P, const RefWinT<WR, WSTEP>& rw, const REF& ref, const LevelDesc& S,
                                               const float* H, int x, int y) {
-    if constexpr (WR > 0) return ncc_cost<WR, WSTEP, PIPE, AHEAD>(P, rw, ref, S, H, x, y);
+    if constexpr (WR > 0) return ncc_cost<WR, WSTEP, PIPE, AHEAD, COPY>(P, rw, ref, S, H, x, y);
     else return ncc_cost_dyn<WSTEP, CHUNK>(P, rw, ref, S, H, x, y);
 }
 

@@ -21,7 +21,8 @@ namespace c3d {
 // its LDS) until its slowest wave is done, and the waves' work differs through the data-dependent
 // early exits.
 constexpr int HALF_SPAN = 128;   // pixel span of one row of 64 active pixels (k_eval of one colour)
-// A wave of the half step takes a block of HALF_BW / TPP x HALF_BH pixels, half of them active. What
+// A wave of the half step takes a block of half_bw x half_bh pixels, half of them active: 16 x 8, or
+// 8 x 8, 8 x 4 and 8 x 2 with two, four and eight lanes per pixel. What
 // a wave costs is what its costliest lane costs, window by window, and pixels of a compact block
 // agree better on it (which sources see them, when a candidate is given up) than 64 pixels along
 // 128 of one row: 3.4 % fewer VALU instructions for the same pixels. The block's samples also share
@@ -29,8 +30,8 @@ constexpr int HALF_SPAN = 128;   // pixel span of one row of 64 active pixels (k
 // staged tile is 2.9 instead of 6.1 KB. 9 views of 1920 x 1080 with 6 sources: half step
 // 23.5 -> 22.2 ms; 2 such views, 3 iterations from a random start: 35.3 -> 31.9 ms; one of
 // 160 x 96: 0.69 -> 0.61 ms.
-constexpr int HALF_BW = 16;
-constexpr int HALF_BH = 8;
+__host__ __device__ constexpr int half_bw(int tpp) { return tpp == 1 ? 16 : 8; }
+__host__ __device__ constexpr int half_bh(int tpp) { return tpp <= 2 ? 8 : 16 / tpp; }
 
 // Active pixel p of a wave's block as (column of active pixels, row): four neighbouring lanes take a
 // 2 x 2 group, so that lanes next to each other sample next to each other in the source, whichever
@@ -49,7 +50,7 @@ __device__ __forceinline__ void block_pixel(int p, int& col, int& row) {
 
 // Pitch of the staged reference rows: the block with its margins, rounded up to 8 modulo 16, with
 // which the 64 lanes of a block read 64 different LDS banks.
-__host__ __device__ constexpr int half_pitch(int tpp, int wr) { return ((HALF_BW / tpp + 2 * wr + 7) / 16) * 16 + 8; }
+__host__ __device__ constexpr int half_pitch(int tpp, int wr) { return ((half_bw(tpp) + 2 * wr + 7) / 16) * 16 + 8; }
 constexpr int PIX_TW = 64;       // eval/filter tiles: 64 x 4 pixels
 constexpr int PIX_TH = 4;
 
@@ -96,7 +97,7 @@ __device__ __forceinline__ TileRefT<WR, TW> tile_ref(const float* tile, int x0, 
 
 // (photometric cost, truncated geometric error) of one hypothesis x one source with the pixel's
 // reciprocal focal lengths hoisted (patchmatch.cu:316-324)
-template <int WR, int WSTEP, bool GEO, int PIPE, bool AHEAD, class REF>
+template <int WR, int WSTEP, bool GEO, int PIPE, bool AHEAD, bool COPY, class REF>
 __device__ __forceinline__ float pair_cost_h(const KParams& P, const RefWinT<WR, WSTEP>& rw, const REF& ref, const LevelDesc& R,
                                              const LevelDesc& S, const PairRec& pr, const LevelPair& lp, float ifx, float ify, int x,
                                              int y, float4 h, float& geo) {
@@ -105,25 +106,41 @@ __device__ __forceinline__ float pair_cost_h(const KParams& P, const RefWinT<WR,
     // geometric runs: the snapshot depth is fetched before the NCC window and used after it
     GeoFetch gf{0.f, 0.f, 0.f, false};
     if constexpr (GEO) gf = geo_fetch(P, R, S, pr, x, y, h.w);
-    if (homography(R, lp, ifx, ify, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP, PIPE, GEO, AHEAD>(P, rw, ref, S, H, x, y);
+    if (homography(R, lp, ifx, ify, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP, PIPE, GEO, AHEAD, COPY>(P, rw, ref, S, H, x, y);
     geo = GEO ? fminf(geo_finish(R, S, pr, x, y, gf), P.gmax) : 0.f;
     return c;
 }
 
 // ================================================================ half step (patchmatch.cu:439-657)
 // GEO: geometric-consistency run (the geometric term is compiled in only there).
-// TPP: lanes per pixel. With 2, the two lanes of a pixel (adjacent lanes) keep their own copies of
-// the pixel's state and split its NCC windows: the step-2 hypotheses by parity and the refinement
-// candidates by parity, exchanging the costs with a lane swap; every decision is then taken on both
-// lanes from the same values in the same order, so the results are those of one lane per pixel.
-template <int WR, int WSTEP, bool GEO, int ROWS, int TPP>
-__global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_half(KParams P) {
+// TPP: lanes per pixel (1, 2, 4 or 8). The lanes of a pixel (neighbours) keep their own copies of the
+// pixel's state and split its NCC windows: lane j of them costs the step-2 hypotheses and the
+// refinement candidates of index j modulo TPP, and the costs are exchanged; every decision is then
+// taken on all of them from the same values in the same order, so the results are those of one
+// lane per pixel.
+// FEW: the build for launches of up to FEW_WAVES waves, at two waves per SIMD, with more gathers in
+// flight and the unrolled copy of the window (see ncc_cost). Its waves are a quarter shorter by
+// themselves, and a launch of a few rounds ends with its last waves: one view of 960 x 540 (4,080
+// waves) takes 2.35 instead of 2.51 ms for 2 iterations with 3 sources, 1920 x 1080 (16,200) 7.33
+// instead of 7.52. Two such views (32,400) tie, and from there the three waves per SIMD of the
+// other build win: 9 views of 1920 x 1080 with 6 sources 22.2 -> 20.0 ms a half step. What binds it
+// is the issue of VALU instructions, which three waves keep busier (3.8 instead of 4.2 cycles an
+// instruction; 2.4 of 3 wave slots taken on average).
+constexpr int FEW_WAVES = 16384;
+template <int WR, int WSTEP>
+constexpr int half_waves(bool few) {
+    return (!few && WR > 0 && Win<(WR > 0 ? WR : 1), WSTEP>::WN2 <= 36) ? 3 : 2;
+}
+
+template <int WR, int WSTEP, bool GEO, int ROWS, int TPP, bool FEW>
+__global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(half_waves<WR, WSTEP>(FEW), half_waves<WR, WSTEP>(FEW))))
+void k_half(KParams P) {
     constexpr int NT = ROWS * 64;
-    constexpr int BW = HALF_BW / TPP, BH = HALF_BH * ROWS;  // pixels of the workgroup's block
-    // source gathers in flight in the window loop: eight where the registers allow (photometric,
-    // one lane per pixel: 247 VGPRs), seven in the geometric build (255), six with two lanes per
-    // pixel, fewer for the 49 register-held weights of a 7 x 7 window (deeper pipelines spill)
-    constexpr int PIPE = Win<(WR > 0 ? WR : 1), WSTEP>::WN2 > 36 ? 3 : (TPP > 1 ? 6 : (GEO ? 7 : 8));
+    constexpr int BW = half_bw(TPP), BH = half_bh(TPP) * ROWS;  // pixels of the workgroup's block
+    // source gathers in flight in the window loop: four for three waves per SIMD (166 VGPRs
+    // photometric; deeper spills and measures no faster), six for two waves, fewer for the 49
+    // register-held weights of a 7 x 7 window
+    constexpr int PIPE = Win<(WR > 0 ? WR : 1), WSTEP>::WN2 > 36 ? 3 : (FEW ? 6 : 4);
     // the reference value of a window sample is read with its gather (see window_sums)
     constexpr bool AHEAD = Win<(WR > 0 ? WR : 1), WSTEP>::WN2 <= 36;
     constexpr int TW = half_pitch(TPP, WR);
@@ -157,7 +174,7 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int sub = lane & (TPP - 1);  // this lane's share of the pixel's windows
     int col, row;
     block_pixel<TPP>(lane / TPP, col, row);
-    const int y = py0 + HALF_BH * (int)(threadIdx.x >> 6) + row;
+    const int y = py0 + half_bh(TPP) * (int)(threadIdx.x >> 6) + row;
     const int x = px0 + 2 * col + ((y + P.color) & 1);
     if (x >= w || y >= h) return;  // both lanes of a pixel leave together
 
@@ -221,9 +238,12 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
     RefWinT<WR, WSTEP> rw;
     ref_stats_any<WR, WSTEP>(P, ref, x, y, wr, rw);
     const int vprev = P.bview[base + pix];
-    float num[9], numf[9];
+    // Aggregated costs: over the adopted sources (weight w2 > 0), or, while none is adopted, the
+    // prior-weighted costs over all sources that the fallback takes. One array holds both in turn:
+    // the first adopted source restarts it, and the fallback is then never used.
+    float agg[9];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) num[i] = numf[i] = 0.f;
+    for (int i = 0; i < 9; ++i) agg[i] = 0.f;
     float den = 0.f, wbest = 0.f, denf = 0.f;
     int vbest = 255;
 #pragma nounroll
@@ -245,7 +265,7 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma nounroll
         for (int i = sub; i < 9; i += TPP) {
             float gi;
-            const float mi = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD>(P, rw, ref, R, S, pr, lp, ifx, ify, x, y, hyp[i * NT], gi);
+            const float mi = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lp, ifx, ify, x, y, hyp[i * NT], gi);
 #pragma unroll
             for (int q = 0; q < 9; ++q)
                 if (q == i) {
@@ -256,11 +276,8 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
         if constexpr (TPP > 1) {
 #pragma unroll
             for (int q = 0; q < 9; ++q) {
-                const float om = __shfl_xor(m[q], 1), og = __shfl_xor(gg[q], 1);
-                if ((q & 1) != sub) {
-                    m[q] = om;
-                    gg[q] = og;
-                }
+                m[q] = __shfl(m[q], lane - sub + (q & (TPP - 1)));
+                if constexpr (GEO) gg[q] = __shfl(gg[q], lane - sub + (q & (TPP - 1)));
             }
         }
         int good = 0, bad = 0;
@@ -278,12 +295,18 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
         float wp = adopt ? (isprev ? 2.f : 1.f) * conf / (float)good : (isprev ? P.prev_w : 0.f);
         float w2 = wp * prior;
         wv[j * P.wv_stride] = w2 > 0.f ? w2 : -prior;
+        const bool adopted = w2 > 0.f;
+        if (adopted && !(den > 0.f)) {
 #pragma unroll
-        for (int i = 0; i < 9; ++i) numf[i] += prior * (m[i] + P.lambda * gg[i]);
+            for (int i = 0; i < 9; ++i) agg[i] = 0.f;
+        }
+        if (adopted || !(den > 0.f)) {
+            const float wa = adopted ? w2 : prior;
+#pragma unroll
+            for (int i = 0; i < 9; ++i) agg[i] += wa * (m[i] + P.lambda * gg[i]);
+        }
         denf += prior;
-        if (w2 > 0.f) {
-#pragma unroll
-            for (int i = 0; i < 9; ++i) num[i] += w2 * (m[i] + P.lambda * gg[i]);
+        if (adopted) {
             den += w2;
             if (w2 > wbest) {
                 wbest = w2;
@@ -291,31 +314,27 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
             }
         }
     }
-    float agg[9];
     int bi9 = 0;
-    if (den > 0.f) {
-#pragma unroll
-        for (int i = 0; i < 9; ++i) agg[i] = num[i] / den;
-#pragma unroll
-        for (int i = 1; i < 9; ++i)
-            if (agg[i] < agg[bi9]) bi9 = i;
-    } else if (denf > 0.f) {
-#pragma unroll
-        for (int i = 0; i < 9; ++i) agg[i] = numf[i] / denf;
-#pragma unroll
-        for (int i = 1; i < 9; ++i)
-            if (agg[i] < agg[bi9]) bi9 = i;
+    const bool fallback = !(den > 0.f) && denf > 0.f;
+    if (fallback) {
         for (int j = 0; j < nsrc; ++j) wv[j * P.wv_stride] = -wv[j * P.wv_stride];
         den = denf;
+    }
+    if (den > 0.f) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) agg[i] = agg[i] / den;
     } else {
 #pragma unroll
         for (int i = 0; i < 9; ++i) agg[i] = 2.f;
     }
-    float4 best = hyp[bi9 * NT];
-    float bcost = 2.f;
+    float bcost = agg[0];
 #pragma unroll
-    for (int q = 0; q < 9; ++q)
-        if (q == bi9) bcost = agg[q];
+    for (int i = 1; i < 9; ++i)
+        if (agg[i] < bcost) {
+            bi9 = i;
+            bcost = agg[i];
+        }
+    float4 best = hyp[bi9 * NT];
 
     // 3. refinement: 6 hypotheses, plus the coarse prior at weak texture (patchmatch.cu:596-653)
     unsigned long long st = rng_state(P.seed, vd.key, P.level, P.run_id, P.t, P.color, (unsigned long long)pix);
@@ -346,9 +365,9 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
     // errors in [0, gmax], lambda >= 0) divided by den: its partial sums only grow, so once
     // nm / den reaches bcost the candidate cannot be accepted and its remaining sources are
     // skipped. The accepted planes and costs are unchanged.
-    // With two lanes per pixel each lane costs every other candidate against the step-2 best (a
+    // With several lanes per pixel each lane costs its candidates against the step-2 best (a
     // candidate that reaches it cannot be accepted later either, the best only decreasing), then
-    // both lanes accept in candidate order from the exchanged costs.
+    // all of them accept in candidate order from the exchanged costs.
     const bool early = P.lambda >= 0.f && (!GEO || P.gmax >= 0.f);
     float ccs[7];
 #pragma unroll
@@ -367,7 +386,7 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
                 const PairRec& pr = prs[j];
                 const LevelDesc S = P.lv[pr.src * P.nlevels + P.level];
                 float g;
-                float m = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD>(P, rw, ref, R, S, pr, lps[j], ifx, ify, x, y, hc, g);
+                float m = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lps[j], ifx, ify, x, y, hc, g);
                 nm += wj * (m + P.lambda * g);
                 if (early && nm / den >= bcost) {
                     out = true;
@@ -389,10 +408,7 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(2, 2)
     }
     if constexpr (TPP > 1) {
 #pragma unroll
-        for (int q = 0; q < 7; ++q) {
-            const float o = __shfl_xor(ccs[q], 1);
-            if ((q & 1) != sub) ccs[q] = o;
-        }
+        for (int q = 0; q < 7; ++q) ccs[q] = __shfl(ccs[q], lane - sub + (q & (TPP - 1)));
 #pragma unroll
         for (int q = 0; q < 7; ++q)
             if (q < ncand && ccs[q] < bcost) {
@@ -883,7 +899,7 @@ __global__ void k_pyramid_step(const uint8_t* src, int w, int h, uint8_t* dst, f
 bool half_shape_ok(int rows, int tpp) { return ((rows == 1 || rows == 2) && tpp == 1) || (rows == 4 && (tpp == 1 || tpp == 2)); }
 
 int half_tiles(const BatchItem* items, int n, int rows, int tpp) {
-    const int bw = HALF_BW / tpp, bh = HALF_BH * rows;
+    const int bw = half_bw(tpp), bh = half_bh(tpp) * rows;
     int t = 0;
     for (int i = 0; i < n; ++i) t += ((items[i].w + bw - 1) / bw) * ((items[i].h + bh - 1) / bh);
     return t;
@@ -900,14 +916,14 @@ int pix_tiles(const BatchItem* items, int n) {
 }
 
 // dynamic LDS bytes of the any-radius (WR = 0) reference tiles
-static size_t half_tile_bytes(int wr, int rows, int tpp) { return (size_t)half_pitch(tpp, wr) * (HALF_BH * rows + 2 * wr) * sizeof(float); }
+static size_t half_tile_bytes(int wr, int rows, int tpp) { return (size_t)half_pitch(tpp, wr) * (half_bh(tpp) * rows + 2 * wr) * sizeof(float); }
 static size_t span_tile_bytes(int wr) { return (size_t)(HALF_SPAN + 2 * wr) * (PIX_TH + 2 * wr) * sizeof(float); }
 static size_t pix_tile_bytes(int wr) { return (size_t)(PIX_TW + 2 * wr) * (PIX_TH + 2 * wr) * sizeof(float); }
 
-template <int WR, int WSTEP, int ROWS, int TPP>
+template <int WR, int WSTEP, int ROWS, int TPP, bool FEW>
 static void launch_half_rows(const KParams& P, size_t lds, hipStream_t s) {
-    if (P.geometric) hipLaunchKernelGGL((k_half<WR, WSTEP, true, ROWS, TPP>), dim3(P.ntiles), dim3(ROWS * 64), lds, s, P);
-    else hipLaunchKernelGGL((k_half<WR, WSTEP, false, ROWS, TPP>), dim3(P.ntiles), dim3(ROWS * 64), lds, s, P);
+    if (P.geometric) hipLaunchKernelGGL((k_half<WR, WSTEP, true, ROWS, TPP, FEW>), dim3(P.ntiles), dim3(ROWS * 64), lds, s, P);
+    else hipLaunchKernelGGL((k_half<WR, WSTEP, false, ROWS, TPP, FEW>), dim3(P.ntiles), dim3(ROWS * 64), lds, s, P);
 }
 
 // P.ntiles must count the tiles of the shape (half_tiles(..., rows, tpp)); the compiled shapes are
@@ -919,10 +935,12 @@ static hipError_t launch_half(const KParams& P0, int rows, int tpp, hipStream_t 
     P.wv_stride = rows * 64;
     size_t lds = (size_t)P.wv_stride * (P.max_nsrc > 0 ? P.max_nsrc : 1) * sizeof(float);
     if (WR == 0) lds += half_tile_bytes(P.wr, rows, tpp);
-    if (rows == 1) launch_half_rows<WR, WSTEP, 1, 1>(P, lds, s);
-    else if (rows == 2) launch_half_rows<WR, WSTEP, 2, 1>(P, lds, s);
-    else if (tpp == 1) launch_half_rows<WR, WSTEP, 4, 1>(P, lds, s);
-    else launch_half_rows<WR, WSTEP, 4, 2>(P, lds, s);
+    const bool few = P.ntiles * rows <= FEW_WAVES;
+    if (rows == 1 && tpp == 1 && few) launch_half_rows<WR, WSTEP, 1, 1, true>(P, lds, s);
+    else if (rows == 1 && tpp == 1) launch_half_rows<WR, WSTEP, 1, 1, false>(P, lds, s);
+    else if (rows == 2) launch_half_rows<WR, WSTEP, 2, 1, false>(P, lds, s);
+    else if (tpp == 1) launch_half_rows<WR, WSTEP, 4, 1, false>(P, lds, s);
+    else launch_half_rows<WR, WSTEP, 4, 2, true>(P, lds, s);
     return hipGetLastError();
 }
 template <int WR, int WSTEP>
@@ -949,7 +967,7 @@ static hipError_t launch_pair_costs(const KParams& P, int view, int slot, int n,
 }
 template <int WR, int WSTEP>
 static const void* half_symbol() {
-    return reinterpret_cast<const void*>(&k_half<WR, WSTEP, false, 4, 1>);
+    return reinterpret_cast<const void*>(&k_half<WR, WSTEP, false, 4, 1, false>);
 }
 
 template <int WR, int WSTEP>
@@ -1063,9 +1081,9 @@ __global__ void k_tile_prefix(const BatchItem* batch, int n, int tw, int th, int
     pre[n] = acc;
 }
 
-// pre: n + 1 ints; the half step's tiles for (rows, lanes per pixel) are HALF_BW / tpp x HALF_BH rows
+// pre: n + 1 ints; the half step's tiles for (rows, lanes per pixel) are half_bw x (half_bh rows)
 hipError_t launch_half_tile_prefix(const BatchItem* batch, int n, int rows, int tpp, int* pre, hipStream_t s) {
-    hipLaunchKernelGGL(k_tile_prefix, dim3(1), dim3(64), 0, s, batch, n, HALF_BW / tpp, HALF_BH * rows, pre);
+    hipLaunchKernelGGL(k_tile_prefix, dim3(1), dim3(64), 0, s, batch, n, half_bw(tpp), half_bh(tpp) * rows, pre);
     return hipGetLastError();
 }
 // the 64 x 4 tiles of k_eval (all pixels) and k_filter (pix_tiles)
