@@ -904,6 +904,19 @@ int half_tiles(const BatchItem* items, int n, int rows, int tpp) {
     for (int i = 0; i < n; ++i) t += ((items[i].w + bw - 1) / bw) * ((items[i].h + bh - 1) / bh);
     return t;
 }
+// Lanes per pixel of a batch when the caller asks for no shape. A launch of few waves lasts as long as
+// one wave does, which is the windows of its pixels one after another: more lanes per pixel make a
+// wave shorter, and cost what every lane repeats of its pixel's own work. Eight or four lanes are
+// taken while the launch stays within one round of two waves per SIMD (2048), two within three rounds.
+// One view with 3 sources, 2 iterations, states in and out, with 8 / 4 / 2 / 1 lanes per pixel:
+// 160 x 96 0.40 / 0.51 / 0.61 / 0.92 ms (before: 0.96), 320 x 180 0.68 / 0.63 / 0.70 / 1.04,
+// 480 x 270 1.16 / 1.00 / 0.90 / 1.13, 760 x 428 2.56 / 2.00 / 1.68 / 1.73, 960 x 540
+// 3.91 / 2.95 / 2.38 / 2.35.
+int half_lanes(const BatchItem* items, int n) {
+    if (half_tiles(items, n, 1, 8) <= 2048) return 8;
+    if (half_tiles(items, n, 1, 4) <= 2048) return 4;
+    return half_tiles(items, n, 1, 2) <= 6144 ? 2 : 1;
+}
 int span_tiles(const BatchItem* items, int n) {
     int t = 0;
     for (int i = 0; i < n; ++i) t += ((items[i].w + HALF_SPAN - 1) / HALF_SPAN) * ((items[i].h + PIX_TH - 1) / PIX_TH);
@@ -927,10 +940,11 @@ static void launch_half_rows(const KParams& P, size_t lds, hipStream_t s) {
 }
 
 // P.ntiles must count the tiles of the shape (half_tiles(..., rows, tpp)); the compiled shapes are
-// (rows, lanes per pixel) = (1, 1), (2, 1), (4, 1) and (4, 2)
+// (rows, lanes per pixel) = (1, 1), (2, 1), (4, 1) and (4, 2), which a caller may ask for, and
+// (1, 2), (1, 4) and (1, 8), which half_lanes picks for small batches
 template <int WR, int WSTEP>
 static hipError_t launch_half(const KParams& P0, int rows, int tpp, hipStream_t s) {
-    if (!half_shape_ok(rows, tpp)) return hipErrorInvalidValue;
+    if (!half_shape_ok(rows, tpp) && !(rows == 1 && (tpp == 2 || tpp == 4 || tpp == 8))) return hipErrorInvalidValue;
     KParams P = P0;
     P.wv_stride = rows * 64;
     size_t lds = (size_t)P.wv_stride * (P.max_nsrc > 0 ? P.max_nsrc : 1) * sizeof(float);
@@ -938,6 +952,9 @@ static hipError_t launch_half(const KParams& P0, int rows, int tpp, hipStream_t 
     const bool few = P.ntiles * rows <= FEW_WAVES;
     if (rows == 1 && tpp == 1 && few) launch_half_rows<WR, WSTEP, 1, 1, true>(P, lds, s);
     else if (rows == 1 && tpp == 1) launch_half_rows<WR, WSTEP, 1, 1, false>(P, lds, s);
+    else if (rows == 1 && tpp == 2) launch_half_rows<WR, WSTEP, 1, 2, true>(P, lds, s);
+    else if (rows == 1 && tpp == 4) launch_half_rows<WR, WSTEP, 1, 4, true>(P, lds, s);
+    else if (rows == 1) launch_half_rows<WR, WSTEP, 1, 8, true>(P, lds, s);
     else if (rows == 2) launch_half_rows<WR, WSTEP, 2, 1, false>(P, lds, s);
     else if (tpp == 1) launch_half_rows<WR, WSTEP, 4, 1, false>(P, lds, s);
     else launch_half_rows<WR, WSTEP, 4, 2, true>(P, lds, s);

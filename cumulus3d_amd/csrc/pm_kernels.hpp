@@ -29,6 +29,8 @@ bool half_shape_ok(int rows, int tpp);
 // workgroup counts of the two tilings for a batch
 int half_tiles(const BatchItem* items, int n, int rows, int tpp);
 int span_tiles(const BatchItem* items, int n);
+// lanes per pixel of the half step for a batch, with one-wave workgroups, when no shape is asked for
+int half_lanes(const BatchItem* items, int n);
 int pix_tiles(const BatchItem* items, int n);
 
 hipError_t launch_sample_reciprocal(const float* z, float* r, long long n, hipStream_t s);

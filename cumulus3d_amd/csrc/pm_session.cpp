@@ -216,6 +216,7 @@ struct c3d_pm_session {
     // options.threads_per_pixel, or c3d_pm_autotune)
     int half_rows = 1;
     int half_tpp = 1;
+    bool half_auto = true;  // neither was given or tuned: every run picks its lanes per pixel (half_lanes)
     // the captured schedule (options.use_graph) and the key it was captured for
     hipGraphExec_t gexec = nullptr;
     std::vector<uint8_t> gkey;
@@ -400,9 +401,10 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
         e.tile_pre = s->tile_pre.p;
         HIP_TRY(s->ks->eval_color(e, st));
     }
-    k.ntiles = half_tiles(items.data(), (int)items.size(), s->half_rows, s->half_tpp);
+    const int tpp = s->half_auto ? half_lanes(items.data(), (int)items.size()) : s->half_tpp;
+    k.ntiles = half_tiles(items.data(), (int)items.size(), s->half_rows, tpp);
     if (iterations > 0) {
-        HIP_TRY(launch_half_tile_prefix(k.batch, k.nitems, s->half_rows, s->half_tpp, s->tile_pre.p, st));
+        HIP_TRY(launch_half_tile_prefix(k.batch, k.nitems, s->half_rows, tpp, s->tile_pre.p, st));
         k.tile_pre = s->tile_pre.p;
     }
     for (uint32_t t = 0; t < iterations; ++t) {
@@ -417,7 +419,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
                 }
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used], st));
             }
-            HIP_TRY(s->ks->half(k, s->half_rows, s->half_tpp, st));
+            HIP_TRY(s->ks->half(k, s->half_rows, tpp, st));
             if (timed) {
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used + 1], st));
                 s->pool_used += 2;
@@ -687,6 +689,7 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     s->filter_copy = fl;
     s->half_tpp = be->opts.threads_per_pixel == 2 ? 2 : 1;
     s->half_rows = default_rows(be->opts.tile_rows, s->half_tpp);
+    s->half_auto = be->opts.tile_rows == 0 && be->opts.threads_per_pixel == 0;
     *out = s;
     return C3D_OK;
 }
@@ -1662,6 +1665,7 @@ int c3d_pm_autotune(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32
     }
     s->half_rows = cand[bestc][0];
     s->half_tpp = cand[bestc][1];
+    s->half_auto = false;
     if (rows_out) *rows_out = (uint32_t)s->half_rows;
     if (tpp_out) *tpp_out = (uint32_t)s->half_tpp;
     if (ms_out)

@@ -58,7 +58,8 @@ typedef struct c3d_pm_options {
     int32_t tile_rows;        /* rows of pixel blocks (one wave each) per half-step workgroup (1, 2 or 4); 0 = 1 (4 with
                                  threads_per_pixel 2) until c3d_pm_autotune */
     int32_t threads_per_pixel;/* lanes per pixel in the half step: 1, or 2 with tile_rows 4 (the two lanes
-                                 split the pixel's NCC windows); 0 = 1 until c3d_pm_autotune */
+                                 split the pixel's NCC windows); 0 = 1 until c3d_pm_autotune, or, with tile_rows 0 too,
+                                 1, 2, 4 or 8 by the pixels of each launch */
     int32_t use_graph;        /* 1 = capture each run's iteration loop in a hipGraph; 0 = plain launches */
     int32_t any_radius;       /* 1 = always the any-radius kernels (weights recomputed per sample), even
                                  for the windows with a register-resident build; 0 = fastest available */

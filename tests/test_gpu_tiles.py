@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
     [(16, 8), (15, 7), (17, 9)],          # one block, one pixel less, one more
     [(31, 33), (8, 64), (240, 8)],        # remainders in both directions, one block high
     [(256, 64), (240, 64), (257, 64)],    # 128, 120 and 136 blocks: a whole round, under it, over it
+    [(161, 119)] * 3,                     # with no shape asked for: four lanes per pixel (eight above)
+    [(255, 161)] * 3,                     # two lanes per pixel
 ])
 def test_block_edges_bit_exact(sizes):
     import oracle
