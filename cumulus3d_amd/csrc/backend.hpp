@@ -6,6 +6,7 @@
 
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/c3d_pm.h"
 
@@ -45,12 +46,24 @@ struct c3d_pm_backend {
     std::mutex life;
     int holders = 0;
     bool destroy_pending = false;
-    // the two page-locked staging buffers of result downloads, used by the session that holds
-    // `lock` and kept for the next one (page-locking hundreds of MB is not free)
+    // the two page-locked staging buffers of result downloads (c3d::download) and the events that
+    // mark them full, used under dl_lock and kept for the next download (page-locking hundreds of MB
+    // is not free)
+    std::mutex dl_lock;
     c3d::PinnedBuf dl_stage[2];
+    hipEvent_t dl_event[2] = {};
 };
 
 namespace c3d {
+// One result array's device source and host destination.
+struct Download {
+    const unsigned char* src;
+    unsigned char* dst;
+    size_t bytes;
+};
+// Copies device arrays, once the work queued on the backend's stream is done, into the caller's
+// (pageable) arrays, and waits for it.
+int download(c3d_pm_backend* be, const std::vector<Download>& xs);
 // Records `msg` as the calling thread's last error (c3d_pm_last_error) and returns `code`.
 int set_error(int code, const std::string& msg);
 // Takes a hold on `be` for a new session or network; fails when c3d_pm_destroy was already called.

@@ -473,44 +473,87 @@ __device__ __forceinline__ float bilin_u8(const uint8_t* g, int w, int h, float 
     return top + ay * (bot - top);
 }
 
-__global__ void k_sweep(SweepArgs a) {
+// One thread per pixel; its 64 bf16 channels leave in eight 16-byte stores.
+__global__ __launch_bounds__(256) void k_sweep(SweepArgs a) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= a.H * a.W) return;
     const int y = i / a.W, x = i - y * a.W;
-    uint16_t* f = a.feat + (long long)i * 64;
-    if (x >= a.rw || y >= a.rh) {
-        for (int c = 0; c < 64; ++c) f[c] = 0;
-        return;
-    }
-    const float ir = a.ref[y * a.rw + x];
+    s16x8* f = (s16x8*)(a.feat + (long long)i * 64);
+    const bool in = x < a.rw && y < a.rh;
+    const float ir = in ? (float)a.ref[y * a.rw + x] : 0.f;
     const float rx = (x - a.rk[2]) / a.rk[0], ry = (y - a.rk[3]) / a.rk[1];
     const float ia = 1.f / a.dmax, ib = 1.f / a.dmin;
-    for (int k = 0; k < 32; ++k) {
-        const float d = 1.f / (ia + (k + 0.5f) / 32.f * (ib - ia));
-        const float X = rx * d, Y = ry * d, Z = d;
-        float cost = 0.f;
-        int n = 0;
-        for (int s = 0; s < a.nsrc; ++s) {
-            const float* R = a.r[s];
-            const float xs = R[0] * X + R[1] * Y + R[2] * Z + a.t[s][0];
-            const float ys = R[3] * X + R[4] * Y + R[5] * Z + a.t[s][1];
-            const float zs = R[6] * X + R[7] * Y + R[8] * Z + a.t[s][2];
-            if (!(zs > 1e-6f)) continue;
-            const float u = a.sk[s][0] * xs / zs + a.sk[s][2], v = a.sk[s][1] * ys / zs + a.sk[s][3];
-            bool inside;
-            const float is = bilin_u8(a.src[s], a.sw[s], a.sh[s], u, v, inside);
-            if (!inside) continue;
-            cost += fabsf(ir - is);
-            n++;
+    for (int k0 = 0; k0 < 32; k0 += 8) {
+        s16x8 o = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (in) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int k = k0 + q;
+                const float d = 1.f / (ia + (k + 0.5f) / 32.f * (ib - ia));
+                const float X = rx * d, Y = ry * d, Z = d;
+                float cost = 0.f;
+                int n = 0;
+                for (int s = 0; s < a.nsrc; ++s) {
+                    const float* R = a.r[s];
+                    const float xs = R[0] * X + R[1] * Y + R[2] * Z + a.t[s][0];
+                    const float ys = R[3] * X + R[4] * Y + R[5] * Z + a.t[s][1];
+                    const float zs = R[6] * X + R[7] * Y + R[8] * Z + a.t[s][2];
+                    if (!(zs > 1e-6f)) continue;
+                    const float u = a.sk[s][0] * xs / zs + a.sk[s][2], v = a.sk[s][1] * ys / zs + a.sk[s][3];
+                    bool inside;
+                    const float is = bilin_u8(a.src[s], a.sw[s], a.sh[s], u, v, inside);
+                    if (!inside) continue;
+                    cost += fabsf(ir - is);
+                    n++;
+                }
+                o[q] = (short)f2bf(n > 0 ? cost / (255.f * n) : 1.f);
+            }
         }
-        f[k] = f2bf(n > 0 ? cost / (255.f * n) : 1.f);
+        f[k0 / 8] = o;
     }
-    f[32] = f2bf(ir / 255.f);
-    for (int c = 33; c < 64; ++c) f[c] = 0;
+    f[4] = s16x8{in ? (short)f2bf(ir / 255.f) : (short)0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int q = 5; q < 8; ++q) f[q] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
 }
 
 hipError_t sweep(const SweepArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_sweep, dim3((unsigned)((a.H * a.W + 255) / 256)), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------- network output -> predictions
+//
+// Bound by the transfer to the host. Formed on the host from the padded 128-byte head output of each
+// pixel, the predictions of 6 images of 480 x 272 took 31 ms of c3d_init_predict; formed here, 40
+// bytes a pixel cross at most, and features and prediction take 3.9 ms together.
+
+__global__ __launch_bounds__(256) void k_predict(PredictArgs a) {
+    const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (p >= a.npix) return;
+    const float4 q = *(const float4*)(a.out + p * 32);
+    const float q4 = a.out[p * 32 + 4];
+    const int b = (int)(p / a.per);
+    const float ia = 1.f / a.range[2 * b + 1], ib = 1.f / a.range[2 * b];
+    if (a.depth) a.depth[p] = 1.f / (ia + 1.f / (1.f + expf(-q.x)) * (ib - ia));
+    if (a.normal) {
+        const float nv = sqrtf(q.y * q.y + q.z * q.z + q.w * q.w + 1e-6f);
+        a.normal[3 * p] = q.y / nv;
+        a.normal[3 * p + 1] = q.z / nv;
+        a.normal[3 * p + 2] = q.w / nv;
+    }
+    if (a.conf) a.conf[p] = 1.f / (1.f + expf(-q4));
+    if (a.head) {
+        float* h = a.head + 5 * p;
+        h[0] = q.x;
+        h[1] = q.y;
+        h[2] = q.z;
+        h[3] = q.w;
+        h[4] = q4;
+    }
+}
+
+hipError_t predict(const PredictArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_predict, dim3((unsigned)((a.npix + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -91,6 +91,16 @@ struct SweepArgs {
 };
 hipError_t sweep(const SweepArgs& a, hipStream_t s);
 
+// Depth, normal (3 floats), confidence and the five head values of every pixel from the network
+// output (each array may be null).
+struct PredictArgs {
+    const float* out;    // head output, [p][32]
+    const float* range;  // [image][2] (depth_min, depth_max)
+    long long npix, per;  // pixels of the batch and of one image
+    float *depth, *normal, *conf, *head;
+};
+hipError_t predict(const PredictArgs& a, hipStream_t s);
+
 // Planes of a full-resolution view from the network output of its quarter-resolution image:
 // inverse depth bilinear, normal and confidence nearest, normal turned towards the camera; depth
 // 0 where the confidence is below `conf_min` (random initialisation there).

@@ -61,6 +61,9 @@ struct c3d_init_net {
     float *g_d0, *g_cat0, *g_d1, *g_cat1, *g_d2, *g_cat2, *g_e3b, *g_e3a, *g_p3, *g_e2b, *g_e2a, *g_p2, *g_e1b, *g_e1a, *g_p1, *g_e0b,
         *g_e0a;
     float *label, *range, *sums;
+    float* pred = nullptr;  // c3d_init_predict's results, from its first call
+    uint8_t* img = nullptr;  // c3d_init_features' images, grown on demand
+    size_t n_img = 0;
     std::vector<float> h_range;
     std::vector<int> h_valid;  // per slot: valid width, height
     int adam_t = 0;
@@ -383,6 +386,7 @@ void c3d_init_destroy(c3d_init_net* n) {
     (void)hipSetDevice(be->device);
     (void)hipStreamSynchronize(be->stream);
     for (void* p : n->allocs) (void)hipFree(p);
+    if (n->img) (void)hipFree(n->img);
     delete n;
     c3d::backend_release(be);
 }
@@ -417,27 +421,50 @@ int c3d_init_features(c3d_init_net* n, uint32_t slot0, uint32_t num, const c3d_s
     if (rc) return rc;
     if (!views || slot0 + num > (uint32_t)n->B) return set_error(C3D_INVALID_ARGUMENT, "slots out of range");
     hipStream_t s = n->be->stream;
-    for (uint32_t i = 0; i < num; ++i) {
+    // every view's images side by side in one kept buffer, so that the views' uploads and sweeps queue
+    // without a wait between them
+    size_t tot = 0;
+    auto room = [](uint32_t w, uint32_t h) { return ((size_t)w * h + 255) & ~(size_t)255; };
+    uint32_t good = 0;  // views before the first bad one: they are done, as if each had its own call
+    int bad = C3D_OK;
+    for (; good < num; ++good) {
+        const c3d_sweep_view& v = views[good];
+        if (!v.gray || v.width > (uint32_t)n->W || v.height > (uint32_t)n->H || v.num_sources < 1 || v.num_sources > 2) {
+            bad = set_error(C3D_INVALID_ARGUMENT, "sweep view larger than the network input or without 1..2 sources");
+            break;
+        }
+        if (!(v.depth_min > 0.f && v.depth_max > v.depth_min)) {
+            bad = set_error(C3D_INVALID_ARGUMENT, "bad depth range");
+            break;
+        }
+        tot += room(v.width, v.height);
+        for (uint32_t j = 0; j < v.num_sources; ++j) tot += room(v.sources[j].width, v.sources[j].height);
+    }
+    if (tot > n->n_img) {
+        if (n->img) {
+            NN_TRY(hipStreamSynchronize(s));
+            (void)hipFree(n->img);
+        }
+        n->img = nullptr;
+        n->n_img = 0;
+        NN_TRY(hipMalloc((void**)&n->img, tot));
+        n->n_img = tot;
+    }
+    hipError_t e = hipSuccess;
+    size_t o = 0;
+    auto put = [&](const uint8_t* src, uint32_t w, uint32_t h) -> const uint8_t* {
+        uint8_t* dst = n->img + o;
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, (size_t)w * h, hipMemcpyHostToDevice, s);
+        o += room(w, h);
+        return dst;
+    };
+    for (uint32_t i = 0; i < good && e == hipSuccess; ++i) {
         const c3d_sweep_view& v = views[i];
-        if (!v.gray || v.width > (uint32_t)n->W || v.height > (uint32_t)n->H || v.num_sources < 1 || v.num_sources > 2)
-            return set_error(C3D_INVALID_ARGUMENT, "sweep view larger than the network input or without 1..2 sources");
-        if (!(v.depth_min > 0.f && v.depth_max > v.depth_min)) return set_error(C3D_INVALID_ARGUMENT, "bad depth range");
-        std::vector<size_t> sz = {(size_t)v.width * v.height};
-        for (uint32_t j = 0; j < v.num_sources; ++j) sz.push_back((size_t)v.sources[j].width * v.sources[j].height);
-        size_t tot = 0;
-        for (size_t z : sz) tot += (z + 255) & ~(size_t)255;
-        uint8_t* img = nullptr;
-        NN_TRY(hipMalloc(&img, tot));
-        size_t o = 0;
         SweepArgs a{};
-        hipError_t e = hipMemcpyAsync(img, v.gray, sz[0], hipMemcpyHostToDevice, s);
-        a.ref = img;
-        o += (sz[0] + 255) & ~(size_t)255;
-        for (uint32_t j = 0; e == hipSuccess && j < v.num_sources; ++j) {
+        a.ref = put(v.gray, v.width, v.height);
+        for (uint32_t j = 0; j < v.num_sources; ++j) {
             const c3d_sweep_source& src = v.sources[j];
-            e = hipMemcpyAsync(img + o, src.gray, sz[j + 1], hipMemcpyHostToDevice, s);
-            a.src[j] = img + o;
-            o += (sz[j + 1] + 255) & ~(size_t)255;
+            a.src[j] = put(src.gray, src.width, src.height);
             a.sw[j] = (int)src.width;
             a.sh[j] = (int)src.height;
             std::memcpy(a.sk[j], src.k, sizeof a.sk[j]);
@@ -454,15 +481,18 @@ int c3d_init_features(c3d_init_net* n, uint32_t slot0, uint32_t num, const c3d_s
         a.H = n->H;
         a.W = n->W;
         if (e == hipSuccess) e = sweep(a, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        (void)hipFree(img);
-        if (e != hipSuccess) return set_error(C3D_DEVICE, std::string("HIP: sweep: ") + hipGetErrorString(e));
-        n->h_range[2 * (slot0 + i)] = v.depth_min;
-        n->h_range[2 * (slot0 + i) + 1] = v.depth_max;
-        n->h_valid[2 * (slot0 + i)] = (int)v.width;
-        n->h_valid[2 * (slot0 + i) + 1] = (int)v.height;
     }
-    return C3D_OK;
+    // the caller's images are free again when this returns
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return set_error(C3D_DEVICE, std::string("HIP: sweep: ") + hipGetErrorString(e));
+    for (uint32_t i = 0; i < good; ++i) {
+        n->h_range[2 * (slot0 + i)] = views[i].depth_min;
+        n->h_range[2 * (slot0 + i) + 1] = views[i].depth_max;
+        n->h_valid[2 * (slot0 + i)] = (int)views[i].width;
+        n->h_valid[2 * (slot0 + i) + 1] = (int)views[i].height;
+    }
+    return bad;
 }
 
 int c3d_init_set_features(c3d_init_net* n, uint32_t num, const uint16_t* feat) {
@@ -555,30 +585,33 @@ int c3d_init_predict(c3d_init_net* n, uint32_t batch, float* depth, float* norma
     int rc = check_net(n);
     if (rc) return rc;
     if (batch < 1 || batch > (uint32_t)n->B) return set_error(C3D_INVALID_ARGUMENT, "batch out of range");
+    hipStream_t s = n->be->stream;
     rc = forward(n, (int)batch);
     if (rc) return rc;
+    // the predictions are formed on the device, so that 40 bytes a pixel cross to the host at most,
+    // not the 128 of the padded head output
     const size_t np = (size_t)batch * n->H * n->W;
-    std::vector<float> o(np * 32);
-    NN_TRY(hipMemcpyAsync(o.data(), n->out32, np * 32 * sizeof(float), hipMemcpyDeviceToHost, n->be->stream));
-    NN_TRY(hipStreamSynchronize(n->be->stream));
-    const size_t per = (size_t)n->H * n->W;
-    for (size_t p = 0; p < np; ++p) {
-        const float* q = &o[p * 32];
-        const size_t b = p / per;
-        const float ia = 1.f / n->h_range[2 * b + 1], ib = 1.f / n->h_range[2 * b];
-        const float s0 = 1.f / (1.f + std::exp(-q[0]));
-        if (depth) depth[p] = 1.f / (ia + s0 * (ib - ia));
-        if (normal) {
-            const float nv = std::sqrt(q[1] * q[1] + q[2] * q[2] + q[3] * q[3] + 1e-6f);
-            normal[3 * p] = q[1] / nv;
-            normal[3 * p + 1] = q[2] / nv;
-            normal[3 * p + 2] = q[3] / nv;
-        }
-        if (conf) conf[p] = 1.f / (1.f + std::exp(-q[4]));
-        if (head)
-            for (int k = 0; k < 5; ++k) head[p * 5 + k] = q[k];
-    }
-    return C3D_OK;
+    if (!n->pred) NN_TRY(alloc(n, &n->pred, (size_t)n->B * n->H * n->W * 10));
+    NN_TRY(hipMemcpyAsync(n->range, n->h_range.data(), (size_t)batch * 2 * sizeof(float), hipMemcpyHostToDevice, s));
+    PredictArgs a{};
+    a.out = n->out32;
+    a.range = n->range;
+    a.npix = (long long)np;
+    a.per = (long long)n->H * n->W;
+    a.depth = depth ? n->pred : nullptr;
+    a.normal = normal ? n->pred + np : nullptr;
+    a.conf = conf ? n->pred + 4 * np : nullptr;
+    a.head = head ? n->pred + 5 * np : nullptr;
+    NN_TRY(predict(a, s));
+    std::vector<c3d::Download> xs;
+    auto add = [&](const float* src, float* dst, size_t count) {
+        if (dst) xs.push_back({(const unsigned char*)src, (unsigned char*)dst, count * sizeof(float)});
+    };
+    add(a.depth, depth, np);
+    add(a.normal, normal, 3 * np);
+    add(a.conf, conf, np);
+    add(a.head, head, 5 * np);
+    return c3d::download(n->be, xs);
 }
 
 }  // extern "C"

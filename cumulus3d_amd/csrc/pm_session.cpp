@@ -130,6 +130,8 @@ namespace {
 void free_backend(c3d_pm_backend* be) {
     (void)hipSetDevice(be->device);
     if (be->stream) (void)hipStreamDestroy(be->stream);
+    for (hipEvent_t e : be->dl_event)
+        if (e) (void)hipEventDestroy(e);
     delete be;
 }
 
@@ -748,7 +750,6 @@ int c3d_pm_run(c3d_pm_session* s, const uint32_t* views, uint32_t n, c3d_view_st
         rc = ensure_snapshot(s, snap, p->level);
         if (rc) return rc;
     }
-    hipStream_t st = s->be->stream;
     for (auto [a, b] : batches(s, views, n, p->level)) {
         std::vector<BatchItem> items;
         long long npix;
@@ -802,10 +803,12 @@ int c3d_pm_evaluate(c3d_pm_session* s, uint32_t level, const uint32_t* views, ui
         KParams k = params_for(s, level, geometric != 0, items, max_nsrc);
         k.ntiles = pix_tiles(items.data(), (int)items.size());
         HIP_TRY(s->ks->eval(k, 0, st));
+        std::vector<c3d::Download> xs;
         for (size_t i = 0; i < items.size(); ++i)
-            HIP_TRY(hipMemcpyAsync(costs[a + i], s->cost.p + items[i].off, (size_t)items[i].w * items[i].h * sizeof(float),
-                                   hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+            xs.push_back({(const unsigned char*)(s->cost.p + items[i].off), (unsigned char*)costs[a + i],
+                          (size_t)items[i].w * items[i].h * sizeof(float)});
+        rc = c3d::download(s->be, xs);
+        if (rc) return rc;
     }
     return C3D_OK;
 }
@@ -832,9 +835,11 @@ int c3d_pm_filter(c3d_pm_session* s, const uint32_t* views, uint32_t n, const c3
         KParams k = params_for(s, level, true, items, max_nsrc);
         k.ntiles = pix_tiles(items.data(), (int)items.size());
         HIP_TRY(s->ks->filter(k, st));
+        std::vector<c3d::Download> xs;
         for (size_t i = 0; i < items.size(); ++i)
-            HIP_TRY(hipMemcpyAsync(counts[a + i], s->count.p + items[i].off, (size_t)items[i].w * items[i].h, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+            xs.push_back({s->count.p + items[i].off, counts[a + i], (size_t)items[i].w * items[i].h});
+        rc = c3d::download(s->be, xs);
+        if (rc) return rc;
     }
     return C3D_OK;
 }
@@ -1458,13 +1463,6 @@ hipError_t grow_temp(c3d_pm_session* s, long long npix) {
     return s->dl_normal.reserve(3 * (size_t)npix);
 }
 
-// One result array's device source and host destination.
-struct Download {
-    const unsigned char* src;
-    unsigned char* dst;
-    size_t bytes;
-};
-
 // A piece of a result array in a staging buffer: its offset there, its destination, its size.
 struct Staged {
     size_t at;
@@ -1510,54 +1508,40 @@ void copy_out(const unsigned char* stage, const std::vector<Staged>& pieces) {
     for (std::thread& x : th) x.join();
 }
 
-// The top-scale results of a densify call copied into the caller's arrays: the planes are split
-// into depth and 3-float normal arrays on the device; then every array goes through two
-// page-locked staging buffers of DL_STAGE bytes: while the device copies into one, host threads
-// copy the other out to the caller's (pageable) arrays.
 constexpr size_t DL_STAGE = 256u << 20;
-int download_states(c3d_pm_session* s, const float4* plane, const float* cost, const BatchItem* items, uint32_t n, long long npix,
-                    c3d_view_state* out, uint8_t* const* counts, float* const* raw_depth) {
-    hipStream_t st = s->be->stream;
-    if (out) {
-        HIP_TRY(grow_temp(s, npix));
-        HIP_TRY(launch_split_planes(plane, s->dl_depth.p, s->dl_normal.p, npix, st));
-    }
-    std::vector<Download> xs;
-    for (uint32_t i = 0; i < n; ++i) {
-        const size_t np = (size_t)items[i].w * items[i].h;
-        const long long off = items[i].off;
-        auto add = [&](const void* src, void* dst, size_t bytes) {
-            if (dst && bytes) xs.push_back({(const unsigned char*)src, (unsigned char*)dst, bytes});
-        };
-        if (out) {
-            add(s->dl_depth.p + off, out[i].depth, np * sizeof(float));
-            add(s->dl_normal.p + 3 * off, out[i].normal, 3 * np * sizeof(float));
-            if (cost) add(cost + off, out[i].cost, np * sizeof(float));
-        }
-        if (raw_depth) add(s->snap.p + off, raw_depth[i], np * sizeof(float));
-        if (counts) add(s->count.p + off, counts[i], np);
-    }
-    if (xs.empty()) {
+}  // namespace
+
+// Every array goes through two page-locked staging buffers: while the device copies into one, host
+// threads copy the other out to the caller's arrays. A buffer holds a quarter of the bytes (1 MiB
+// at least, DL_STAGE at most), so that small results overlap too and page-lock little.
+int c3d::download(c3d_pm_backend* be, const std::vector<Download>& xs) {
+    hipStream_t st = be->stream;
+    size_t total = 0;
+    for (const Download& x : xs) total += x.bytes;
+    if (total == 0) {
         HIP_TRY(hipStreamSynchronize(st));
         return C3D_OK;
     }
+    std::lock_guard<std::mutex> g(be->dl_lock);
+    size_t stage_bytes = std::min(DL_STAGE, std::max<size_t>((total / 4 + 4095) & ~(size_t)4095, 1u << 20));
     // $C3D_PM_STAGE_BYTES (64 bytes or more) shrinks the staging buffers, so that tests can switch
     // between them many times on small jobs
-    size_t stage_bytes = DL_STAGE;
     if (const char* e = std::getenv("C3D_PM_STAGE_BYTES")) {
         const long long v = std::atoll(e);
-        if (v >= 64 && (size_t)v < DL_STAGE) stage_bytes = (size_t)v;
+        if (v >= 64 && (size_t)v < stage_bytes) stage_bytes = (size_t)v;
     }
-    PinnedBuf* stage = s->be->dl_stage;
-    HIP_TRY(stage[0].reserve(stage_bytes));
-    HIP_TRY(stage[1].reserve(stage_bytes));
+    PinnedBuf* stage = be->dl_stage;
+    for (int b = 0; b < 2; ++b) {
+        HIP_TRY(stage[b].reserve(stage_bytes));
+        if (!be->dl_event[b]) HIP_TRY(hipEventCreateWithFlags(&be->dl_event[b], hipEventDisableTiming));
+    }
     std::vector<Staged> staged[2];
     bool busy[2] = {false, false};
     int cur = 0;
     size_t fill = 0;
     auto drain = [&](int b) -> hipError_t {
         if (!busy[b]) return hipSuccess;
-        hipError_t e = hipEventSynchronize(s->ev[6 + b]);
+        hipError_t e = hipEventSynchronize(be->dl_event[b]);
         if (e != hipSuccess) return e;
         copy_out(stage[b].p, staged[b]);
         staged[b].clear();
@@ -1565,7 +1549,7 @@ int download_states(c3d_pm_session* s, const float4* plane, const float* cost, c
         return hipSuccess;
     };
     auto close_buffer = [&]() -> hipError_t {  // the device copies into `cur` are queued: switch
-        hipError_t e = hipEventRecord(s->ev[6 + cur], st);
+        hipError_t e = hipEventRecord(be->dl_event[cur], st);
         if (e != hipSuccess) return e;
         busy[cur] = true;
         cur = 1 - cur;
@@ -1587,6 +1571,34 @@ int download_states(c3d_pm_session* s, const float4* plane, const float* cost, c
     HIP_TRY(drain(0));
     HIP_TRY(drain(1));
     return C3D_OK;
+}
+
+namespace {
+// The results of a call copied into the caller's arrays: the planes are split into depth and
+// 3-float normal arrays on the device, then every array is downloaded.
+int download_states(c3d_pm_session* s, const float4* plane, const float* cost, const BatchItem* items, uint32_t n, long long npix,
+                    c3d_view_state* out, uint8_t* const* counts, float* const* raw_depth) {
+    hipStream_t st = s->be->stream;
+    if (out) {
+        HIP_TRY(grow_temp(s, npix));
+        HIP_TRY(launch_split_planes(plane, s->dl_depth.p, s->dl_normal.p, npix, st));
+    }
+    std::vector<c3d::Download> xs;
+    for (uint32_t i = 0; i < n; ++i) {
+        const size_t np = (size_t)items[i].w * items[i].h;
+        const long long off = items[i].off;
+        auto add = [&](const void* src, void* dst, size_t bytes) {
+            if (dst && bytes) xs.push_back({(const unsigned char*)src, (unsigned char*)dst, bytes});
+        };
+        if (out) {
+            add(s->dl_depth.p + off, out[i].depth, np * sizeof(float));
+            add(s->dl_normal.p + 3 * off, out[i].normal, 3 * np * sizeof(float));
+            if (cost) add(cost + off, out[i].cost, np * sizeof(float));
+        }
+        if (raw_depth) add(s->snap.p + off, raw_depth[i], np * sizeof(float));
+        if (counts) add(s->count.p + off, counts[i], np);
+    }
+    return c3d::download(s->be, xs);
 }
 
 int download_results(c3d_pm_session* s, const BatchItem* items, uint32_t n, long long npix, c3d_view_state* out,
