@@ -2,10 +2,8 @@
 // accumulation on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16), its backward pass, Adam,
 // the training loss against plain-PatchStereo labels and the plane-sweep input features.
 //
-// Convolutions are implicit GEMMs over NHWC tensors: the 64 lanes of a wave load 16 pixels x 32
-// channels (one 16-byte load per lane) as an A operand and 32 channels x 16 output channels of
-// the weights as the B operand, which serves the wave's 1 or 4 groups of 16 pixels; a 256-thread
-// workgroup computes 64 or 256 pixels x 64 output channels.
+// Convolutions are implicit GEMMs over NHWC tensors: a workgroup stages a tile of pixels with its
+// halo in LDS, from where its four waves read the pixels of every tap as one MFMA operand; the weights, packed in the order the lanes take them, come from L2 as the other.
 // The weight gradient stages 32 pixels x 32 channels of both operands transposed in LDS so that
 // the reduction over pixels is the MFMA's K dimension.
 #include "nn_kernels.hpp"
@@ -14,6 +12,7 @@ namespace c3d {
 namespace nn {
 
 typedef short s16x8 __attribute__((__vector_size__(16)));
+typedef short s16x4 __attribute__((__vector_size__(8)));
 typedef float f32x4 __attribute__((__vector_size__(16)));
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -30,100 +29,141 @@ __device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) { return __buil
 
 // ---------------------------------------------------------------- convolution (forward / data gradient)
 
-// G pixel groups of 16 per wave: the wave loads each B operand (32 input x 16 output channels of
-// one tap) once for its G groups. Every output still accumulates tap by tap and 32 channels at a
-// time in the same order, so G changes no result.
-template <int G>
+// A workgroup computes 16 x 4R pixels x 16 NT output channels: wave w the rows w R .. w R + R - 1. It
+// stages the tile and its halo, all input channels (groups of 32 one after another, so that the 64
+// lanes read 64 bytes a pixel without bank conflicts). The weights are the MFMA's first operand, so
+// that a lane ends with four channels of one pixel and stores them at once; those of the next step
+// are loaded while a step's are used. Every output accumulates tap by tap and 32 channels at a
+// time in the same order, so R and NT change no result.
+//
+// What bounds it: the layers are small (0.3 to 15 GFLOP), so the latency of the staging and the
+// stores count as much as the matrix cores; at R = 4, NT = 4 these could be kept half busy by LDS
+// and fully by L1. Reading each tap's pixels from L1 instead, 16 or 64 pixels a wave, left them at
+// 130 TFLOP/s: the forward pass of 6 images of 480 x 272 took 1.48 ms of convolutions, now 0.60 (350
+// TFLOP/s), a training step of 8 images 3.70, now 1.25.
+template <int KS, int R, int NT>
 __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
+    constexpr int HALO = KS / 2, TAPS = KS * KS;
+    constexpr int TW = 16 + 2 * HALO, TH = 4 * R + 2 * HALO, NPX = TW * TH;
+    constexpr int NLD = (NPX * 4 + 255) / 256;  // 16-byte loads a thread per 32 channels
+    extern __shared__ __attribute__((aligned(16))) uint16_t tile[];  // [cin / 32][NPX][32]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kg = lane >> 4;
-    const long long HW = (long long)a.H * a.W;
-    const long long P = (long long)a.nimg * HW;
-    const long long p0 = ((long long)blockIdx.x * 4 + wave) * (16 * G);
-    const int co0 = blockIdx.y * 64;
-    const int ntile = min(4, (a.cout - co0) / 16);
-    int img[G], py[G], px[G];
-    bool pin[G];
+    const int tx = (a.W + 15) / 16, ty = (a.H + 4 * R - 1) / (4 * R);
+    const int img = (int)(blockIdx.x / (unsigned)(tx * ty)), rest = (int)(blockIdx.x % (unsigned)(tx * ty));
+    const int y0 = rest / tx * (4 * R), x0 = rest % tx * 16;
+    const int ct0 = blockIdx.y * NT;
+    const int nc = a.cin / 32;
+    {
+        int pix[NLD];  // the pixel of each of this thread's loads, -1 outside the image
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const long long pa = p0 + 16 * g + r16;
-        pin[g] = pa < P;
-        img[g] = py[g] = px[g] = 0;
-        if (pin[g]) {
-            img[g] = (int)(pa / HW);
-            const int rem = (int)(pa - (long long)img[g] * HW);
-            py[g] = rem / a.W;
-            px[g] = rem - py[g] * a.W;
+        for (int j = 0; j < NLD; ++j) {
+            const int e = threadIdx.x + 256 * j, p = e >> 2;
+            const int gy = y0 + p / TW - HALO, gx = x0 + p % TW - HALO;
+            pix[j] = (e < NPX * 4 && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W) ? (img * a.H + gy) * a.W + gx : -1;
         }
-    }
-    f32x4 acc[G][4];
+#pragma unroll 2
+        for (int c = 0; c < nc; ++c) {
+            s16x8 v[NLD];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int taps = a.ksize * a.ksize, rad = a.ksize / 2;
-    for (int t = 0; t < taps; ++t) {
-        const int dy = t / a.ksize - rad, dx = t % a.ksize - rad;
-        bool ok[G];
-        long long xoff[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int qy = py[g] + dy, qx = px[g] + dx;
-            ok[g] = pin[g] && qy >= 0 && qy < a.H && qx >= 0 && qx < a.W;
-            xoff[g] = ok[g] ? (((long long)img[g] * HW + (long long)qy * a.W + qx) * a.xs + kg * 8) : 0;
-        }
-        for (int c0 = 0; c0 < a.cin; c0 += 32) {
-            s16x8 A[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                A[g] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-                if (ok[g]) A[g] = *(const s16x8*)(a.x + xoff[g] + c0);
+            for (int j = 0; j < NLD; ++j) {
+                v[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                if (pix[j] >= 0) v[j] = *(const s16x8*)(a.x + (size_t)pix[j] * a.xs + c * 32 + (threadIdx.x & 3) * 8);
             }
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt) {
-                if (tt < ntile) {
-                    const int co = co0 + tt * 16 + r16;
-                    const s16x8 B = *(const s16x8*)(a.w + ((long long)co * taps + t) * a.cin + c0 + kg * 8);
-#pragma unroll
-                    for (int g = 0; g < G; ++g) acc[g][tt] = mfma(A[g], B, acc[g][tt]);
-                }
-            }
+            for (int j = 0; j < NLD; ++j)
+                if ((int)threadIdx.x + 256 * j < NPX * 4) *(s16x8*)&tile[(size_t)c * NPX * 32 + (threadIdx.x + 256 * j) * 8] = v[j];
         }
     }
-    // lane holds rows (pixels) 4 kg + j and column (output channel) r16 of each 16 x 16 tile
+    f32x4 acc[R][NT];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-            if (tt >= ntile) continue;
-            const int co = co0 + tt * 16 + r16;
-            const float b = a.bias ? a.bias[co] : 0.f;
+        for (int n = 0; n < NT; ++n) acc[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint16_t* w = a.w + (size_t)ct0 * 512 + lane * 8;
+    s16x8 wn[NT];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long long p = p0 + 16 * g + 4 * kg + j;
-                if (p >= P) continue;
-                float v = acc[g][tt][j] + b;
-                if (a.mode == 0) {
-                    if (a.relu) v = fmaxf(v, 0.f);
-                    a.y[p * a.ys + a.yoff + co] = f2bf(v);
-                } else if (a.mode == 1) {
-                    a.y32[p * a.y32s + co] = v;
-                } else {
-                    a.y32[p * a.y32s + co] += v;
+    for (int n = 0; n < NT; ++n) wn[n] = *(const s16x8*)(w + n * 512);
+    __syncthreads();
+    int left = TAPS * nc;
+    for (int dy = 0; dy < KS; ++dy)
+        for (int dx = 0; dx < KS; ++dx) {
+            const uint16_t* t = tile + ((wave * R + dy) * TW + r16 + dx) * 32 + kg * 8;
+#pragma unroll 1
+            for (int c = 0; c < nc; ++c, t += NPX * 32) {
+                s16x8 X[R], wc[NT];
+#pragma unroll
+                for (int r = 0; r < R; ++r) X[r] = *(const s16x8*)(t + r * TW * 32);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) wc[n] = wn[n];
+                if (--left > 0) {
+                    w += (size_t)a.ctiles * 512;
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) wn[n] = *(const s16x8*)(w + n * 512);
                 }
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r][n] = mfma(wc[n], X[r], acc[r][n]);
+            }
+        }
+    // lane holds pixel r16 of each row and channels 4 kg .. 4 kg + 3 of each 16
+    const int x = x0 + r16;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int co = (ct0 + n) * 16 + 4 * kg;
+        const f32x4 b = a.bias ? *(const f32x4*)(a.bias + co) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = y0 + wave * R + r;
+            if (x >= a.W || y >= a.H) continue;
+            const size_t p = (size_t)(img * a.H + y) * a.W + x;
+            f32x4 v = acc[r][n] + b;
+            if (a.y32) {
+                *(f32x4*)(a.y32 + p * a.y32s + co) = v;
+            } else {
+                s16x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = (short)f2bf(a.relu ? fmaxf(v[j], 0.f) : v[j]);
+                *(s16x4*)(a.y + p * a.ys + co) = o;
             }
         }
     }
 }
 
-// Four pixel groups per wave where the launch still has at least 512 workgroups (two per CU),
-// one otherwise (the small deep layers keep their parallelism).
+template <int KS, int R, int NT>
+static void launch_conv_rows(const ConvArgs& a, unsigned blocks, unsigned ny, size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL((k_conv<KS, R, NT>), dim3(blocks, ny), dim3(256), lds, s, a);
+}
+
+// Taller tiles stage less halo and use each weight for more pixels; smaller ones are taken where a
+// launch would otherwise have fewer than two workgroups per CU, or one CU's LDS no room for two.
+template <int KS, int NT>
+static void launch_conv(const ConvArgs& a, hipStream_t s) {
+    const unsigned tx = (unsigned)((a.W + 15) / 16), ny = (unsigned)(a.cout / (16 * NT));
+    auto blocks = [&](int rows) { return (unsigned)a.nimg * tx * (unsigned)((a.H + rows - 1) / rows); };
+    auto lds = [&](int rows) { return (size_t)(16 + 2 * (KS / 2)) * (rows + 2 * (KS / 2)) * a.cin * sizeof(uint16_t); };
+    auto good = [&](int rows) { return blocks(rows) * ny >= 512 && lds(rows) <= 80 * 1024; };
+    if (good(16)) launch_conv_rows<KS, 4, NT>(a, blocks(16), ny, lds(16), s);
+    else if (good(8)) launch_conv_rows<KS, 2, NT>(a, blocks(8), ny, lds(8), s);
+    else launch_conv_rows<KS, 1, NT>(a, blocks(4), ny, lds(4), s);
+}
+
+// cout: 16 or a multiple of 32; 16 NT channels a workgroup
 hipError_t conv(const ConvArgs& a, hipStream_t s) {
-    const long long P = (long long)a.nimg * a.H * a.W;
-    const unsigned ny = (unsigned)((a.cout + 63) / 64);
-    const long long n4 = (P + 255) / 256;
-    if (n4 * ny >= 512) hipLaunchKernelGGL(k_conv<4>, dim3((unsigned)n4, ny), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(k_conv<1>, dim3((unsigned)((P + 63) / 64), ny), dim3(256), 0, s, a);
+    if (a.cin % 32 != 0 || a.cin > 256 || (a.cout != 16 && a.cout % 32 != 0) || (a.ksize != 1 && a.ksize != 3)) return hipErrorInvalidValue;
+    if (a.ksize == 1) {
+        if (a.cout == 16) launch_conv<1, 1>(a, s);
+        else launch_conv<1, 2>(a, s);
+    } else if (a.cout % 64 == 0) {
+        launch_conv<3, 4>(a, s);
+    } else if (a.cout % 96 == 0) {
+        launch_conv<3, 6>(a, s);
+    } else if (a.cout % 32 == 0) {
+        launch_conv<3, 2>(a, s);
+    } else {
+        return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
@@ -351,6 +391,12 @@ hipError_t fill(float* p, float v, long long n, hipStream_t s) {
     return hipGetLastError();
 }
 
+// A convolution's weights in the order k_conv reads them: for each tap, 32 input channels and 16
+// output channels the 64 lanes' 8 values (lane = 16 (ci % 32 / 8) + co % 16).
+__device__ __forceinline__ size_t packed(int ci, int t, int co, int cin, int cout) {
+    return ((((size_t)t * (cin / 32) + ci / 32) * (cout / 16) + co / 16) * 64 + (ci % 32 / 8) * 16 + co % 16) * 8 + ci % 8;
+}
+
 __global__ void k_weights_bf16(const float* w32, int cout, int taps, int cin, uint16_t* w, uint16_t* wt) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long n = (long long)cout * taps * cin;
@@ -359,9 +405,9 @@ __global__ void k_weights_bf16(const float* w32, int cout, int taps, int cin, ui
     const int t = (int)((i / cin) % taps);
     const int co = (int)(i / ((long long)cin * taps));
     const uint16_t b = f2bf(w32[i]);
-    w[i] = b;
-    // data gradient: wt[ci][taps - 1 - t][co]
-    wt[((long long)ci * taps + (taps - 1 - t)) * cout + co] = b;
+    w[packed(ci, t, co, cin, cout)] = b;
+    // data gradient: the taps flipped, input and output channels exchanged
+    wt[packed(co, taps - 1 - t, ci, cout, cin)] = b;
 }
 
 hipError_t weights_bf16(const float* w32, int cout, int taps, int cin, uint16_t* w, uint16_t* wt, hipStream_t s) {

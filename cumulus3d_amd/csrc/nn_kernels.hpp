@@ -17,14 +17,15 @@ struct ConvArgs {
     const uint16_t* x;
     int xs, cin;  // channel stride and count of the input (cin a multiple of 32)
     int nimg, H, W, ksize;
-    const uint16_t* w;  // [cout][ksize * ksize][cin]
+    const uint16_t* w;  // packed by weights_bf16
     const float* bias;  // [cout] or null
-    int cout;           // a multiple of 16
-    uint16_t* y;        // mode 0: bf16 output at channel offset yoff of a tensor with stride ys
-    int ys, yoff;
-    float* y32;  // modes 1 and 2: fp32 output with stride y32s (1: store, 2: accumulate)
+    int cout;           // 16 or a multiple of 32: the output channels computed
+    int ctiles;         // 16-channel groups in `w` (those of all its output channels)
+    uint16_t* y;        // bf16 output with channel stride ys, when y32 is null
+    int ys;
+    float* y32;  // fp32 output with channel stride y32s
     int y32s;
-    int mode, relu;
+    int relu;  // bf16 output only
 };
 
 // Weight gradient dw[co][tap][ci] += sum_p dz[p][co] * x[p + off(tap)][ci] (fp32 atomics).
@@ -55,7 +56,7 @@ hipError_t copy_channels(const uint16_t* x, int xs, int c, long long npix, uint1
 hipError_t add_channels(const float* dy, int dys, int off, int c, long long npix, float* dx, int dxs, hipStream_t s);
 // fp32 fill
 hipError_t fill(float* p, float v, long long n, hipStream_t s);
-// weight layout transforms: bf16 forward copy and the flipped, transposed data-gradient copy
+// weights in bf16, packed for conv: the forward copy and the flipped, transposed data-gradient copy
 hipError_t weights_bf16(const float* w32, int cout, int taps, int cin, uint16_t* w, uint16_t* wt, hipStream_t s);
 
 // Loss of the 5 head outputs against plain-PatchStereo labels, and its gradient (bf16, stride 32).

@@ -28,8 +28,8 @@ struct Layer {
     int cin, cout, k, relu;
     int cin_real;  // input channels that carry data (fan-in of the initialisation)
     size_t woff, boff;
-    uint16_t* w = nullptr;   // [cout][k*k][cin] bf16
-    uint16_t* wt = nullptr;  // [cin][k*k][cout] bf16, taps flipped (data gradient)
+    uint16_t* w = nullptr;   // bf16, packed for conv (weights_bf16)
+    uint16_t* wt = nullptr;  // the same for the data gradient, taps flipped
 };
 
 enum { E0A, E0B, E1A, E1B, E2A, E2B, E3A, E3B, D2, D1, D0, HEAD, NLAYER };
@@ -104,13 +104,12 @@ int conv_fwd(c3d_init_net* n, int li, const uint16_t* x, int nimg, int h, int w,
     a.ksize = l.k;
     a.w = l.w;
     a.bias = n->w32 + l.boff;
-    a.cout = l.cout;
+    a.cout = y32 ? 16 : l.cout;  // the head: 5 of its 32 padded outputs are used
+    a.ctiles = l.cout / 16;
     a.y = y;
     a.ys = l.cout;
-    a.yoff = 0;
     a.y32 = y32;
     a.y32s = l.cout;
-    a.mode = y32 ? 1 : 0;
     a.relu = l.relu;
     NN_TRY(conv(a, n->be->stream));
     return C3D_OK;
@@ -177,9 +176,9 @@ int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, in
         a.w = l.wt;
         a.bias = nullptr;
         a.cout = l.cin;
+        a.ctiles = l.cin / 16;
         a.y32 = dx;
         a.y32s = l.cin;
-        a.mode = 1;
         NN_TRY(conv(a, s));
     }
     return C3D_OK;
