@@ -8,6 +8,8 @@
 // the reduction over pixels is the MFMA's K dimension.
 #include "nn_kernels.hpp"
 
+#include <algorithm>
+
 namespace c3d {
 namespace nn {
 
@@ -242,39 +244,55 @@ hipError_t wgrad(const WgradArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-__global__ void k_bias_grad(const uint16_t* dz, int dzs, int c, long long npix, float* db) {
-    const int ch = blockIdx.y * 64 + (threadIdx.x & 63);
-    if (ch >= c) return;
-    const long long p0 = (long long)blockIdx.x * WG_CHUNK;
-    const long long p1 = min(npix, p0 + WG_CHUNK);
-    float acc = 0.f;
-    for (long long p = p0 + (threadIdx.x >> 6); p < p1; p += 4) acc += bf2f(dz[p * dzs + ch]);
-    atomicAdd(&db[ch], acc);
+// dz = bf16(da * (a > 0)) and db[c] += sum_p dz[p][c]; without `da`, dz is given and only summed. One
+// workgroup takes DZ_CHUNK pixels, a thread 8 channels of every (2048 / c)th of them; the workgroup's
+// sums are added up in LDS before one atomic per channel. Bound by HBM: 8 bytes a value. As two
+// passes, with one value a thread and every thread of the second walking 1,024 pixels two bytes at a
+// time, they took 3.36 ms of a training step on 8 images of 480 x 272, now 0.46.
+constexpr int DZ_CHUNK = 1024;
+
+template <bool RELU>
+__global__ __launch_bounds__(256) void k_dz(const float* da, const uint16_t* a, uint16_t* dz, int c, long long npix, float* db) {
+    __shared__ float sum[256 * 8];
+    const int groups = c / 8, g = threadIdx.x % groups, pstep = 256 / groups;
+    const long long p0 = (long long)blockIdx.x * DZ_CHUNK, p1 = min(npix, p0 + DZ_CHUNK);
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if ((int)threadIdx.x < pstep * groups)
+        for (long long p = p0 + threadIdx.x / groups; p < p1; p += pstep) {
+            const size_t i = (size_t)p * c + g * 8;
+            s16x8 z;
+            if constexpr (RELU) {
+                const s16x8 av = *(const s16x8*)(a + i);
+                const f32x4 d0 = *(const f32x4*)(da + i), d1 = *(const f32x4*)(da + i + 4);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) z[j] = (short)f2bf(bf2f((uint16_t)av[j]) > 0.f ? (j < 4 ? d0[j & 3] : d1[j & 3]) : 0.f);
+                *(s16x8*)(dz + i) = z;
+            } else {
+                z = *(const s16x8*)(dz + i);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] += bf2f((uint16_t)z[j]);
+        }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[threadIdx.x * 8 + j] = acc[j];
+    __syncthreads();
+    for (int ch = threadIdx.x; ch < c; ch += 256) {
+        float s = 0.f;
+        for (int q = 0; q < pstep; ++q) s += sum[(q * groups + ch / 8) * 8 + (ch & 7)];
+        atomicAdd(&db[ch], s);
+    }
 }
 
-hipError_t bias_grad(const uint16_t* dz, int dzs, int c, long long npix, float* db, hipStream_t s) {
-    dim3 grid((unsigned)((npix + WG_CHUNK - 1) / WG_CHUNK), (unsigned)((c + 63) / 64));
-    hipLaunchKernelGGL(k_bias_grad, grid, dim3(256), 0, s, dz, dzs, c, npix, db);
+// c: a multiple of 32, at most 2048; da and a null: dz is given
+hipError_t dz_grad(const float* da, const uint16_t* a, uint16_t* dz, int c, long long npix, float* db, hipStream_t s) {
+    if (c % 32 != 0 || c > 2048 || (da == nullptr) != (a == nullptr)) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)((npix + DZ_CHUNK - 1) / DZ_CHUNK);
+    if (da) hipLaunchKernelGGL(k_dz<true>, dim3(blocks), dim3(256), 0, s, da, a, dz, c, npix, db);
+    else hipLaunchKernelGGL(k_dz<false>, dim3(blocks), dim3(256), 0, s, da, a, dz, c, npix, db);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- elementwise and resampling
-
-__global__ void k_relu_grad(const float* da, int das, const uint16_t* a, int as, uint16_t* dz, int dzs, int c, long long n) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n * c) return;
-    const long long p = i / c;
-    const int ch = (int)(i - p * c);
-    const float g = bf2f(a[p * as + ch]) > 0.f ? da[p * das + ch] : 0.f;
-    dz[p * dzs + ch] = f2bf(g);
-}
-
-hipError_t relu_grad(const float* da, int das, const uint16_t* a, int as, uint16_t* dz, int dzs, int c, long long npix,
-                     hipStream_t s) {
-    const long long n = npix * c;
-    hipLaunchKernelGGL(k_relu_grad, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, da, das, a, as, dz, dzs, c, npix);
-    return hipGetLastError();
-}
 
 __global__ void k_pool(const uint16_t* x, int xs, int c, int nimg, int H, int W, uint16_t* y, int ys) {
     const int Ho = H / 2, Wo = W / 2;
@@ -426,12 +444,17 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__global__ void k_loss(LossArgs a) {
-    const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
+// The four sums leave a workgroup in one atomic each, from at most LOSS_BLOCKS workgroups: atomics of
+// every wave on the same four words took 0.83 ms of a training step on 8 images of 480 x 272
+// (0.04 now).
+constexpr int LOSS_BLOCKS = 512;
+
+__global__ __launch_bounds__(256) void k_loss(LossArgs a) {
+    __shared__ float part[4][4];
     const long long HW = (long long)a.H * a.W;
     const long long P = a.nimg * HW;
     float ld = 0.f, ln = 0.f, lc = 0.f, cnt = 0.f;
-    if (p < P) {
+    for (long long p = (long long)blockIdx.x * 256 + threadIdx.x; p < P; p += (long long)gridDim.x * 256) {
         float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
         const int b = (int)(p / HW);
         const int rem = (int)(p - (long long)b * HW);
@@ -444,21 +467,21 @@ __global__ void k_loss(LossArgs a) {
             const float id = ia + s0 * (ib - ia);
             const float idt = 1.f / lb[0];
             const float e = id - idt;
-            ld = fabsf(e) / (ib - ia);
+            ld += fabsf(e) / (ib - ia);
             g[0] = (e > 0.f ? 1.f : (e < 0.f ? -1.f : 0.f)) * s0 * (1.f - s0);
             const float vx = o[1], vy = o[2], vz = o[3];
             const float nv = sqrtf(vx * vx + vy * vy + vz * vz + 1e-6f);
             const float nx = vx / nv, ny = vy / nv, nz = vz / nv;
             const float dot = nx * lb[1] + ny * lb[2] + nz * lb[3];
-            ln = 1.f - dot;
+            ln += 1.f - dot;
             g[1] = -a.w_normal * (lb[1] - dot * nx) / nv;
             g[2] = -a.w_normal * (lb[2] - dot * ny) / nv;
             g[3] = -a.w_normal * (lb[3] - dot * nz) / nv;
             const float c = sigm(o[4]);
             const float tgt = fabsf(1.f / id - lb[0]) <= a.conf_tol * lb[0] ? 1.f : 0.f;
-            lc = -(tgt * __logf(fmaxf(c, 1e-7f)) + (1.f - tgt) * __logf(fmaxf(1.f - c, 1e-7f)));
+            lc += -(tgt * __logf(fmaxf(c, 1e-7f)) + (1.f - tgt) * __logf(fmaxf(1.f - c, 1e-7f)));
             g[4] = a.w_conf * (c - tgt);
-            cnt = 1.f;
+            cnt += 1.f;
         }
         uint16_t* d = a.dout + p * 32;
 #pragma unroll
@@ -469,16 +492,19 @@ __global__ void k_loss(LossArgs a) {
     lc = wave_sum(lc);
     cnt = wave_sum(cnt);
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&a.sums[0], ld);
-        atomicAdd(&a.sums[1], ln);
-        atomicAdd(&a.sums[2], lc);
-        atomicAdd(&a.sums[3], cnt);
+        float* q = part[threadIdx.x >> 6];
+        q[0] = ld;
+        q[1] = ln;
+        q[2] = lc;
+        q[3] = cnt;
     }
+    __syncthreads();
+    if (threadIdx.x < 4) atomicAdd(&a.sums[threadIdx.x], part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x]);
 }
 
 hipError_t loss(const LossArgs& a, hipStream_t s) {
     const long long P = (long long)a.nimg * a.H * a.W;
-    hipLaunchKernelGGL(k_loss, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_loss, dim3((unsigned)std::min<long long>((P + 255) / 256, LOSS_BLOCKS)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -40,11 +40,8 @@ struct WgradArgs {
 
 hipError_t conv(const ConvArgs& a, hipStream_t s);
 hipError_t wgrad(const WgradArgs& a, hipStream_t s);
-// db[c] += sum_p dz[p][c]
-hipError_t bias_grad(const uint16_t* dz, int dzs, int c, long long npix, float* db, hipStream_t s);
-// dz = bf16(da * (a > 0)) over c channels
-hipError_t relu_grad(const float* da, int das, const uint16_t* a, int as, uint16_t* dz, int dzs, int c, long long npix,
-                     hipStream_t s);
+// dz = bf16(da * (a > 0)) over [npix][c] and db[c] += sum_p dz[p][c]; with da and a null dz is given
+hipError_t dz_grad(const float* da, const uint16_t* a, uint16_t* dz, int c, long long npix, float* db, hipStream_t s);
 // 2x2 mean pooling (H, W even) and its gradient (accumulated)
 hipError_t pool(const uint16_t* x, int xs, int c, int nimg, int H, int W, uint16_t* y, int ys, hipStream_t s);
 hipError_t pool_grad(const float* dy, int dys, int c, int nimg, int H, int W, float* dx, int dxs, hipStream_t s);

@@ -144,8 +144,8 @@ int forward(c3d_init_net* n, int b) {
     return C3D_OK;
 }
 
-// Gradient of a layer from the gradient at its (pre-activation) output dz: weights, bias, and
-// (when dx is given) the input gradient, stored.
+// Gradient of a layer from the gradient at its (pre-activation) output dz: weights and (when dx is
+// given) the input gradient, stored.
 int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, int nimg, int h, int w, float* dx) {
     const Layer& l = n->L[li];
     hipStream_t s = n->be->stream;
@@ -162,8 +162,6 @@ int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, in
     g.ksize = l.k;
     g.dw = n->g32 + l.woff;
     NN_TRY(wgrad(g, s));
-    const long long np = (long long)nimg * h * w;
-    NN_TRY(bias_grad(dz, l.cout, l.cout, np, n->g32 + l.boff, s));
     if (dx) {
         ConvArgs a{};
         a.x = dz;
@@ -184,11 +182,11 @@ int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, in
     return C3D_OK;
 }
 
-// dz = relu'(a) * da, then the layer's gradients
+// dz = relu'(a) * da with its sums (the bias gradient), then the layer's other gradients
 int relu_layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* a, const float* da, int nimg, int h, int w, float* dx) {
     const Layer& l = n->L[li];
     const long long np = (long long)nimg * h * w;
-    NN_TRY(relu_grad(da, l.cout, a, l.cout, n->dz, l.cout, l.cout, np, n->be->stream));
+    NN_TRY(dz_grad(da, a, n->dz, l.cout, np, n->g32 + l.boff, n->be->stream));
     return layer_bwd(n, li, x, n->dz, nimg, h, w, dx);
 }
 
@@ -205,6 +203,7 @@ int backward(c3d_init_net* n, int b) {
     NN_TRY(fill(n->g_e1b, 0.f, P1 * 64, s));
     NN_TRY(fill(n->g_e0b, 0.f, P0 * 32, s));
     // head (no activation): dz = dout
+    NN_TRY(dz_grad(nullptr, nullptr, n->dout, n->L[HEAD].cout, P0, n->g32 + n->L[HEAD].boff, s));
     if ((rc = layer_bwd(n, HEAD, n->d0, n->dout, b, H, W, n->g_d0))) return rc;
     if ((rc = relu_layer_bwd(n, D0, n->cat0, n->d0, n->g_d0, b, H, W, n->g_cat0))) return rc;
     NN_TRY(upsample_grad(n->g_cat0, 96, 0, 64, b, H / 2, W / 2, n->g_d1, 64, s));
