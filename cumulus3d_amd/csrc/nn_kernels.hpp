@@ -13,9 +13,11 @@ namespace nn {
 
 // Convolution (3x3 or 1x1, stride 1, zero padding) as an implicit GEMM on MFMA:
 // y[p][co] = sum_{tap, ci} x[p + off(tap)][ci] * w[co][tap][ci].
+// The input is x (channels 0 .. c1 - 1, its channel stride) followed by x2 (the other cin - c1, null
+// when there are none); with `up`, x has half the size and is upsampled by repetition.
 struct ConvArgs {
-    const uint16_t* x;
-    int xs, cin;  // channel stride and count of the input (cin a multiple of 32)
+    const uint16_t *x, *x2;
+    int c1, cin, up;  // multiples of 32
     int nimg, H, W, ksize;
     const uint16_t* w;  // packed by weights_bf16
     const float* bias;  // [cout] or null
@@ -28,28 +30,30 @@ struct ConvArgs {
     int relu;  // bf16 output only
 };
 
-// Weight gradient dw[co][tap][ci] += sum_p dz[p][co] * x[p + off(tap)][ci] (fp32 atomics).
+// Weight gradient dw[co][tap][ci] = sum_p dz[p][co] * x[p + off(tap)][ci], x as in ConvArgs.
 struct WgradArgs {
-    const uint16_t* x;
-    int xs, cin;
+    const uint16_t *x, *x2;
+    int c1, cin, up;
     const uint16_t* dz;
-    int dzs, cout;
+    int cout;
     int nimg, H, W, ksize;
     float* dw;
 };
+// The workspace of partial sums holds wgrad_slices(a) times the layer's weights, at most
+// WG_SLICE_FLOATS floats.
+constexpr long long WG_SLICE_FLOATS = 10ll << 20;
+int wgrad_slices(const WgradArgs& a);
 
 hipError_t conv(const ConvArgs& a, hipStream_t s);
-hipError_t wgrad(const WgradArgs& a, hipStream_t s);
+hipError_t wgrad(const WgradArgs& a, float* slices, hipStream_t s);
 // dz = bf16(da * (a > 0)) over [npix][c] and db[c] += sum_p dz[p][c]; with da and a null dz is given
 hipError_t dz_grad(const float* da, const uint16_t* a, uint16_t* dz, int c, long long npix, float* db, hipStream_t s);
 // 2x2 mean pooling (H, W even) and its gradient (accumulated)
 hipError_t pool(const uint16_t* x, int xs, int c, int nimg, int H, int W, uint16_t* y, int ys, hipStream_t s);
 hipError_t pool_grad(const float* dy, int dys, int c, int nimg, int H, int W, float* dx, int dxs, hipStream_t s);
-// nearest 2x upsampling of x (nimg, H, W) into channels [yoff, yoff + c) of y (nimg, 2H, 2W)
-hipError_t upsample(const uint16_t* x, int xs, int c, int nimg, int H, int W, uint16_t* y, int ys, int yoff, hipStream_t s);
+// gradient of the nearest 2x upsampling of c channels of dy from channel yoff (accumulated)
 hipError_t upsample_grad(const float* dy, int dys, int yoff, int c, int nimg, int H, int W, float* dx, int dxs, hipStream_t s);
-// y[:, yoff : yoff + c] = x ; dx += dy[:, off : off + c]
-hipError_t copy_channels(const uint16_t* x, int xs, int c, long long npix, uint16_t* y, int ys, int yoff, hipStream_t s);
+// dx += dy[:, off : off + c]
 hipError_t add_channels(const float* dy, int dys, int off, int c, long long npix, float* dx, int dxs, hipStream_t s);
 // fp32 fill
 hipError_t fill(float* p, float v, long long n, hipStream_t s);

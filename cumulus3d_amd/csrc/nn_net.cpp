@@ -56,11 +56,12 @@ struct c3d_init_net {
     size_t nparam = 0;
     float *w32 = nullptr, *g32 = nullptr, *m32 = nullptr, *v32 = nullptr;
     // activations (bf16) and their gradients (fp32)
-    uint16_t *feat, *e0a, *e0b, *p1, *e1a, *e1b, *p2, *e2a, *e2b, *p3, *e3a, *e3b, *cat2, *d2, *cat1, *d1, *cat0, *d0, *dout, *dz;
+    uint16_t *feat, *e0a, *e0b, *p1, *e1a, *e1b, *p2, *e2a, *e2b, *p3, *e3a, *e3b, *d2, *d1, *d0, *dout, *dz;
     float* out32;
     float *g_d0, *g_cat0, *g_d1, *g_cat1, *g_d2, *g_cat2, *g_e3b, *g_e3a, *g_p3, *g_e2b, *g_e2a, *g_p2, *g_e1b, *g_e1a, *g_p1, *g_e0b,
         *g_e0a;
     float *label, *range, *sums;
+    float* slices = nullptr;  // partial weight gradients, from the first training step
     float* pred = nullptr;  // c3d_init_predict's results, from its first call
     uint8_t* img = nullptr;  // c3d_init_features' images, grown on demand
     size_t n_img = 0;
@@ -92,12 +93,20 @@ int upload_weights(c3d_init_net* n) {
     return C3D_OK;
 }
 
-int conv_fwd(c3d_init_net* n, int li, const uint16_t* x, int nimg, int h, int w, uint16_t* y, float* y32) {
+// The input of a layer: x, or x at half the size (upsampled) followed by the skip's channels.
+struct In {
+    const uint16_t *x, *x2 = nullptr;
+    int c2 = 0;
+};
+
+int conv_fwd(c3d_init_net* n, int li, In in, int nimg, int h, int w, uint16_t* y, float* y32) {
     const Layer& l = n->L[li];
     ConvArgs a{};
-    a.x = x;
-    a.xs = l.cin;
+    a.x = in.x;
+    a.x2 = in.x2;
+    a.c1 = l.cin - in.c2;
     a.cin = l.cin;
+    a.up = in.x2 != nullptr;
     a.nimg = nimg;
     a.H = h;
     a.W = w;
@@ -119,54 +128,47 @@ int forward(c3d_init_net* n, int b) {
     hipStream_t s = n->be->stream;
     const int H = n->H, W = n->W;
     int rc;
-    if ((rc = conv_fwd(n, E0A, n->feat, b, H, W, n->e0a, nullptr))) return rc;
-    if ((rc = conv_fwd(n, E0B, n->e0a, b, H, W, n->e0b, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E0A, In{n->feat}, b, H, W, n->e0a, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E0B, In{n->e0a}, b, H, W, n->e0b, nullptr))) return rc;
     NN_TRY(pool(n->e0b, 32, 32, b, H, W, n->p1, 32, s));
-    if ((rc = conv_fwd(n, E1A, n->p1, b, H / 2, W / 2, n->e1a, nullptr))) return rc;
-    if ((rc = conv_fwd(n, E1B, n->e1a, b, H / 2, W / 2, n->e1b, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E1A, In{n->p1}, b, H / 2, W / 2, n->e1a, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E1B, In{n->e1a}, b, H / 2, W / 2, n->e1b, nullptr))) return rc;
     NN_TRY(pool(n->e1b, 64, 64, b, H / 2, W / 2, n->p2, 64, s));
-    if ((rc = conv_fwd(n, E2A, n->p2, b, H / 4, W / 4, n->e2a, nullptr))) return rc;
-    if ((rc = conv_fwd(n, E2B, n->e2a, b, H / 4, W / 4, n->e2b, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E2A, In{n->p2}, b, H / 4, W / 4, n->e2a, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E2B, In{n->e2a}, b, H / 4, W / 4, n->e2b, nullptr))) return rc;
     NN_TRY(pool(n->e2b, 128, 128, b, H / 4, W / 4, n->p3, 128, s));
-    if ((rc = conv_fwd(n, E3A, n->p3, b, H / 8, W / 8, n->e3a, nullptr))) return rc;
-    if ((rc = conv_fwd(n, E3B, n->e3a, b, H / 8, W / 8, n->e3b, nullptr))) return rc;
-    const long long P0 = (long long)b * H * W, P1 = P0 / 4, P2 = P0 / 16;
-    NN_TRY(upsample(n->e3b, 128, 128, b, H / 8, W / 8, n->cat2, 256, 0, s));
-    NN_TRY(copy_channels(n->e2b, 128, 128, P2, n->cat2, 256, 128, s));
-    if ((rc = conv_fwd(n, D2, n->cat2, b, H / 4, W / 4, n->d2, nullptr))) return rc;
-    NN_TRY(upsample(n->d2, 128, 128, b, H / 4, W / 4, n->cat1, 192, 0, s));
-    NN_TRY(copy_channels(n->e1b, 64, 64, P1, n->cat1, 192, 128, s));
-    if ((rc = conv_fwd(n, D1, n->cat1, b, H / 2, W / 2, n->d1, nullptr))) return rc;
-    NN_TRY(upsample(n->d1, 64, 64, b, H / 2, W / 2, n->cat0, 96, 0, s));
-    NN_TRY(copy_channels(n->e0b, 32, 32, P0, n->cat0, 96, 64, s));
-    if ((rc = conv_fwd(n, D0, n->cat0, b, H, W, n->d0, nullptr))) return rc;
-    if ((rc = conv_fwd(n, HEAD, n->d0, b, H, W, nullptr, n->out32))) return rc;
+    if ((rc = conv_fwd(n, E3A, In{n->p3}, b, H / 8, W / 8, n->e3a, nullptr))) return rc;
+    if ((rc = conv_fwd(n, E3B, In{n->e3a}, b, H / 8, W / 8, n->e3b, nullptr))) return rc;
+    if ((rc = conv_fwd(n, D2, In{n->e3b, n->e2b, 128}, b, H / 4, W / 4, n->d2, nullptr))) return rc;
+    if ((rc = conv_fwd(n, D1, In{n->d2, n->e1b, 64}, b, H / 2, W / 2, n->d1, nullptr))) return rc;
+    if ((rc = conv_fwd(n, D0, In{n->d1, n->e0b, 32}, b, H, W, n->d0, nullptr))) return rc;
+    if ((rc = conv_fwd(n, HEAD, In{n->d0}, b, H, W, nullptr, n->out32))) return rc;
     return C3D_OK;
 }
 
 // Gradient of a layer from the gradient at its (pre-activation) output dz: weights and (when dx is
 // given) the input gradient, stored.
-int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, int nimg, int h, int w, float* dx) {
+int layer_bwd(c3d_init_net* n, int li, In in, const uint16_t* dz, int nimg, int h, int w, float* dx) {
     const Layer& l = n->L[li];
     hipStream_t s = n->be->stream;
     WgradArgs g{};
-    g.x = x;
-    g.xs = l.cin;
+    g.x = in.x;
+    g.x2 = in.x2;
+    g.c1 = l.cin - in.c2;
     g.cin = l.cin;
+    g.up = in.x2 != nullptr;
     g.dz = dz;
-    g.dzs = l.cout;
     g.cout = l.cout;
     g.nimg = nimg;
     g.H = h;
     g.W = w;
     g.ksize = l.k;
     g.dw = n->g32 + l.woff;
-    NN_TRY(wgrad(g, s));
+    NN_TRY(wgrad(g, n->slices, s));
     if (dx) {
         ConvArgs a{};
         a.x = dz;
-        a.xs = l.cout;
-        a.cin = l.cout;
+        a.c1 = a.cin = l.cout;
         a.nimg = nimg;
         a.H = h;
         a.W = w;
@@ -183,11 +185,11 @@ int layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* dz, in
 }
 
 // dz = relu'(a) * da with its sums (the bias gradient), then the layer's other gradients
-int relu_layer_bwd(c3d_init_net* n, int li, const uint16_t* x, const uint16_t* a, const float* da, int nimg, int h, int w, float* dx) {
+int relu_layer_bwd(c3d_init_net* n, int li, In in, const uint16_t* a, const float* da, int nimg, int h, int w, float* dx) {
     const Layer& l = n->L[li];
     const long long np = (long long)nimg * h * w;
     NN_TRY(dz_grad(da, a, n->dz, l.cout, np, n->g32 + l.boff, n->be->stream));
-    return layer_bwd(n, li, x, n->dz, nimg, h, w, dx);
+    return layer_bwd(n, li, in, n->dz, nimg, h, w, dx);
 }
 
 int backward(c3d_init_net* n, int b) {
@@ -204,27 +206,27 @@ int backward(c3d_init_net* n, int b) {
     NN_TRY(fill(n->g_e0b, 0.f, P0 * 32, s));
     // head (no activation): dz = dout
     NN_TRY(dz_grad(nullptr, nullptr, n->dout, n->L[HEAD].cout, P0, n->g32 + n->L[HEAD].boff, s));
-    if ((rc = layer_bwd(n, HEAD, n->d0, n->dout, b, H, W, n->g_d0))) return rc;
-    if ((rc = relu_layer_bwd(n, D0, n->cat0, n->d0, n->g_d0, b, H, W, n->g_cat0))) return rc;
+    if ((rc = layer_bwd(n, HEAD, In{n->d0}, n->dout, b, H, W, n->g_d0))) return rc;
+    if ((rc = relu_layer_bwd(n, D0, In{n->d1, n->e0b, 32}, n->d0, n->g_d0, b, H, W, n->g_cat0))) return rc;
     NN_TRY(upsample_grad(n->g_cat0, 96, 0, 64, b, H / 2, W / 2, n->g_d1, 64, s));
     NN_TRY(add_channels(n->g_cat0, 96, 64, 32, P0, n->g_e0b, 32, s));
-    if ((rc = relu_layer_bwd(n, D1, n->cat1, n->d1, n->g_d1, b, H / 2, W / 2, n->g_cat1))) return rc;
+    if ((rc = relu_layer_bwd(n, D1, In{n->d2, n->e1b, 64}, n->d1, n->g_d1, b, H / 2, W / 2, n->g_cat1))) return rc;
     NN_TRY(upsample_grad(n->g_cat1, 192, 0, 128, b, H / 4, W / 4, n->g_d2, 128, s));
     NN_TRY(add_channels(n->g_cat1, 192, 128, 64, P1, n->g_e1b, 64, s));
-    if ((rc = relu_layer_bwd(n, D2, n->cat2, n->d2, n->g_d2, b, H / 4, W / 4, n->g_cat2))) return rc;
+    if ((rc = relu_layer_bwd(n, D2, In{n->e3b, n->e2b, 128}, n->d2, n->g_d2, b, H / 4, W / 4, n->g_cat2))) return rc;
     NN_TRY(upsample_grad(n->g_cat2, 256, 0, 128, b, H / 8, W / 8, n->g_e3b, 128, s));
     NN_TRY(add_channels(n->g_cat2, 256, 128, 128, P2, n->g_e2b, 128, s));
-    if ((rc = relu_layer_bwd(n, E3B, n->e3a, n->e3b, n->g_e3b, b, H / 8, W / 8, n->g_e3a))) return rc;
-    if ((rc = relu_layer_bwd(n, E3A, n->p3, n->e3a, n->g_e3a, b, H / 8, W / 8, n->g_p3))) return rc;
+    if ((rc = relu_layer_bwd(n, E3B, In{n->e3a}, n->e3b, n->g_e3b, b, H / 8, W / 8, n->g_e3a))) return rc;
+    if ((rc = relu_layer_bwd(n, E3A, In{n->p3}, n->e3a, n->g_e3a, b, H / 8, W / 8, n->g_p3))) return rc;
     NN_TRY(pool_grad(n->g_p3, 128, 128, b, H / 4, W / 4, n->g_e2b, 128, s));
-    if ((rc = relu_layer_bwd(n, E2B, n->e2a, n->e2b, n->g_e2b, b, H / 4, W / 4, n->g_e2a))) return rc;
-    if ((rc = relu_layer_bwd(n, E2A, n->p2, n->e2a, n->g_e2a, b, H / 4, W / 4, n->g_p2))) return rc;
+    if ((rc = relu_layer_bwd(n, E2B, In{n->e2a}, n->e2b, n->g_e2b, b, H / 4, W / 4, n->g_e2a))) return rc;
+    if ((rc = relu_layer_bwd(n, E2A, In{n->p2}, n->e2a, n->g_e2a, b, H / 4, W / 4, n->g_p2))) return rc;
     NN_TRY(pool_grad(n->g_p2, 64, 64, b, H / 2, W / 2, n->g_e1b, 64, s));
-    if ((rc = relu_layer_bwd(n, E1B, n->e1a, n->e1b, n->g_e1b, b, H / 2, W / 2, n->g_e1a))) return rc;
-    if ((rc = relu_layer_bwd(n, E1A, n->p1, n->e1a, n->g_e1a, b, H / 2, W / 2, n->g_p1))) return rc;
+    if ((rc = relu_layer_bwd(n, E1B, In{n->e1a}, n->e1b, n->g_e1b, b, H / 2, W / 2, n->g_e1a))) return rc;
+    if ((rc = relu_layer_bwd(n, E1A, In{n->p1}, n->e1a, n->g_e1a, b, H / 2, W / 2, n->g_p1))) return rc;
     NN_TRY(pool_grad(n->g_p1, 32, 32, b, H, W, n->g_e0b, 32, s));
-    if ((rc = relu_layer_bwd(n, E0B, n->e0a, n->e0b, n->g_e0b, b, H, W, n->g_e0a))) return rc;
-    if ((rc = relu_layer_bwd(n, E0A, n->feat, n->e0a, n->g_e0a, b, H, W, nullptr))) return rc;
+    if ((rc = relu_layer_bwd(n, E0B, In{n->e0a}, n->e0b, n->g_e0b, b, H, W, n->g_e0a))) return rc;
+    if ((rc = relu_layer_bwd(n, E0A, In{n->feat}, n->e0a, n->g_e0a, b, H, W, nullptr))) return rc;
     return C3D_OK;
 }
 
@@ -313,11 +315,8 @@ int c3d_init_create(c3d_pm_backend* be, uint32_t max_batch, uint32_t height, uin
     A(n->p3, P3 * 128);
     A(n->e3a, P3 * 128);
     A(n->e3b, P3 * 128);
-    A(n->cat2, P2 * 256);
     A(n->d2, P2 * 128);
-    A(n->cat1, P1 * 192);
     A(n->d1, P1 * 64);
-    A(n->cat0, P0 * 96);
     A(n->d0, P0 * 32);
     A(n->dout, P0 * 32);
     A(n->dz, P0 * 32);
@@ -544,6 +543,7 @@ int c3d_init_train_step(c3d_init_net* n, uint32_t batch, const c3d_init_train_pa
         if (n->h_valid[2 * i] != n->h_valid[0] || n->h_valid[2 * i + 1] != n->h_valid[1])
             return set_error(C3D_INVALID_ARGUMENT, "every slot of a batch needs the same valid size");
     hipStream_t s = n->be->stream;
+    if (!n->slices) NN_TRY(alloc(n, &n->slices, (size_t)WG_SLICE_FLOATS));
     NN_TRY(hipMemcpyAsync(n->range, n->h_range.data(), (size_t)batch * 2 * sizeof(float), hipMemcpyHostToDevice, s));
     rc = forward(n, (int)batch);
     if (rc) return rc;

@@ -32,3 +32,32 @@ def test_conv_tile_edges(batch, h, w):
     err = np.abs(head[0] - out[0])
     assert err.max() <= 0.02 * np.abs(out).max() and err.mean() <= 0.002 * np.abs(out).max()
     be.close()
+
+
+@pytest.mark.parametrize("batch,h,w", [(3, 8, 8), (4, 40, 72), (17, 24, 40)])
+def test_weight_gradient_tiles_and_slices(batch, h, w):
+    """The gradient reduces tiles of 32 x 16 pixels into slices by the number of tiles; the convolutions
+    give an image the same bits in any batch, so a batch's gradients are its images' summed (fp32
+    sums: 1e-5 relative)."""
+    from oracle import nn_oracle as nno
+
+    rng = np.random.default_rng(9)
+    feat = np.zeros((batch, h, w, 64), np.float32)
+    feat[..., :33] = rng.uniform(0, 1, (batch, h, w, 33))
+    bits = nno.bf16_bits(feat)
+    depth = rng.uniform(20, 60, (batch, h, w)).astype(np.float32)
+    normal = np.tile(np.float32([0.1, -0.2, -0.97]), (batch, h, w, 1))
+    be = pm.HipPatchMatch()
+    big, one = (init_net.InitNet(be, n, h, w, seed=11) for n in (batch, 1))
+    big.set_features(bits)
+    total = np.zeros(big.n)
+    for b in range(batch):
+        big.set_labels(b, depth[b], normal[b], w - 3, h - 2, 15.0, 120.0)
+        one.set_features(bits[b : b + 1])
+        one.set_labels(0, depth[b], normal[b], w - 3, h - 2, 15.0, 120.0)
+        total += one.train_step(1, init_net.TrainParams(), step=False, want_grads=True)[1]
+    got = big.train_step(batch, init_net.TrainParams(), step=False, want_grads=True)[1]
+    for name, woff, boff, cin, cout, k, relu in nno.layout()[0]:
+        for lo, hi in ((woff, boff), (boff, boff + cout)):
+            assert np.linalg.norm(got[lo:hi] - total[lo:hi]) <= 1e-5 * np.linalg.norm(total[lo:hi]), name
+    be.close()
