@@ -34,6 +34,8 @@ struct LevelDesc {
     long long qoff;  // dword offset of quad entry (0, 0) (the 2-texel border precedes it)
     long long goff;  // byte offset of the u8 image
     float fx, fy, cx, cy;
+    float ifx, ify;   // 1 / fx, 1 / fy
+    int plain, pad1;  // both focal lengths lie where division by them may go through div_exact
 };
 
 struct PairRec {
@@ -243,6 +245,27 @@ __device__ __forceinline__ float rcp_sample(float z) {
     return r;
 }
 
+// Correctly rounded 1/x, a/b and square root from the hardware estimates and FMA residuals (Newton's
+// step, and Markstein's: q + (a - b q) y rounds to a/b when y is the rounded 1/b and q within an ulp),
+// the same bits as IEEE division and sqrtf in 3, 3 and 5 instructions; the compiler's sequences,
+// which also serve the ends of the exponent range, take 10, 10 and 13. inv_exact and sqrt_exact equal
+// the IEEE results on every mantissa of one and of two binades (measured on the device). For
+// arguments and results between 2^-100 and 2^100; callers keep IEEE division for the rest.
+__device__ __forceinline__ float inv_exact(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fmaf(r, fmaf(-x, r, 1.0f), r);
+}
+__device__ __forceinline__ float div_exact(float a, float b, float inv_b) {
+    const float q = a * inv_b;
+    return fmaf(fmaf(-b, q, a), inv_b, q);
+}
+__device__ __forceinline__ float sqrt_exact(float x) {
+    const float r = __builtin_amdgcn_rsqf(x);
+    const float s = x * r;
+    return fmaf(fmaf(-s, s, x), 0.5f * r, s);
+}
+constexpr float EXACT_LO = 0x1p-100f, EXACT_HI = 0x1p100f;
+
 // ---------------------------------------------------------------- vectors
 
 struct f3 {
@@ -359,7 +382,14 @@ __device__ __forceinline__ bool homography(const LevelDesc& R, const LevelPair& 
     f3 ray = mk3((x - R.cx) * ifx, (y - R.cy) * ify, 1.0f);
     float delta = d * dot3(n, ray);
     if (!(delta < -1e-12f)) return false;
-    float id = 1.0f / delta, invd = 1.0f / d;
+    float id, invd;
+    if (fmaxf(-delta, fabsf(d)) < EXACT_HI && fabsf(d) > EXACT_LO) {
+        id = inv_exact(delta);
+        invd = inv_exact(d);
+    } else {
+        id = 1.0f / delta;
+        invd = 1.0f / d;
+    }
     float u0 = n.x * ifx, u1 = n.y * ify;
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
@@ -567,10 +597,11 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
                                           const float* H, int x, int y) {
     float z = H[8];
     if (!(z > 1e-8f)) return 2.0f;
-    float iz = 1.0f / z;
-    float u = H[2] * iz;
-    float v = H[5] * iz;
-    if (!(u >= 0.f && v >= 0.f && u <= (float)(S.w - 1) && v <= (float)(S.h - 1))) return 2.0f;
+    const float iz = z < EXACT_HI ? inv_exact(z) : 1.0f / z;
+    const float u = H[2] * iz;
+    const float v = H[5] * iz;
+    // inside the source (a NaN position is not)
+    if (!(__builtin_amdgcn_fmed3f(u, 0.f, (float)(S.w - 1)) == u && __builtin_amdgcn_fmed3f(v, 0.f, (float)(S.h - 1)) == v)) return 2.0f;
     if (rw.var < P.vmin255) return 2.0f;
     const uint32_t* qbase = P.quad + (S.qoff - 2LL * S.qpitch - 2);
     const float qp4 = 4.0f * (float)S.qpitch, koff4 = 2.0f * qp4 + 8.0f;
@@ -592,7 +623,9 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
     float vars = fmaf(-mus, mus, SSs * iW);
     if (vars < P.vmin255) return 2.0f;
     float cov = fmaf(-rw.mu, mus, IS * iW);
-    float cc = 1.0f - cov / sqrtf(rw.var * vars);
+    // both variances lie between vmin255 and 255^2; a quotient below the exact range vanishes from 1 - rho
+    const float sd = sqrt_exact(rw.var * vars);
+    float cc = 1.0f - div_exact(cov, sd, inv_exact(sd));
     return fminf(fmaxf(cc, 0.0f), 2.0f);
 }
 
@@ -656,10 +689,11 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
                               int y) {
     float z = H[8];
     if (!(z > 1e-8f)) return 2.0f;
-    float iz = 1.0f / z;
-    float u = H[2] * iz;
-    float v = H[5] * iz;
-    if (!(u >= 0.f && v >= 0.f && u <= (float)(S.w - 1) && v <= (float)(S.h - 1))) return 2.0f;
+    const float iz = z < EXACT_HI ? inv_exact(z) : 1.0f / z;
+    const float u = H[2] * iz;
+    const float v = H[5] * iz;
+    // inside the source (a NaN position is not)
+    if (!(__builtin_amdgcn_fmed3f(u, 0.f, (float)(S.w - 1)) == u && __builtin_amdgcn_fmed3f(v, 0.f, (float)(S.h - 1)) == v)) return 2.0f;
     if (rw.var < P.vmin255) return 2.0f;
     const uint32_t* qbase = P.quad + (S.qoff - 2LL * S.qpitch - 2);
     const float qp4 = 4.0f * (float)S.qpitch, koff4 = 2.0f * qp4 + 8.0f;
@@ -734,7 +768,9 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
     float vars = fmaf(-mus, mus, SSs * iW);
     if (vars < P.vmin255) return 2.0f;
     float cov = fmaf(-rw.mu, mus, IS * iW);
-    float cc = 1.0f - cov / sqrtf(rw.var * vars);
+    // both variances lie between vmin255 and 255^2; a quotient below the exact range vanishes from 1 - rho
+    const float sd = sqrt_exact(rw.var * vars);
+    float cc = 1.0f - div_exact(cov, sd, inv_exact(sd));
     return fminf(fmaxf(cc, 0.0f), 2.0f);
 }
 
@@ -772,7 +808,15 @@ __device__ __forceinline__ GeoFetch geo_fetch(const KParams& P, const LevelDesc&
     float yj = pr.r[3] * X.x + pr.r[4] * X.y + pr.r[5] * X.z + pr.t[1];
     float zj = pr.r[6] * X.x + pr.r[7] * X.y + pr.r[8] * X.z + pr.t[2];
     if (!(zj > 1e-8f)) return g;
-    float u = S.fx * xj / zj + S.cx, v = S.fy * yj / zj + S.cy;
+    float u, v;
+    if (zj < EXACT_HI) {
+        const float iz = inv_exact(zj);
+        u = div_exact(S.fx * xj, zj, iz) + S.cx;
+        v = div_exact(S.fy * yj, zj, iz) + S.cy;
+    } else {
+        u = S.fx * xj / zj + S.cx;
+        v = S.fy * yj / zj + S.cy;
+    }
     float uf = floorf(u + 0.5f), vf = floorf(v + 0.5f);
     if (!(uf >= 0.f && vf >= 0.f && uf < (float)S.w && vf < (float)S.h)) return g;
     g.dj = P.snap[off + (long long)vf * S.w + (long long)uf];
@@ -786,13 +830,23 @@ __device__ __forceinline__ float geo_finish(const LevelDesc& R, const LevelDesc&
     if (!g.ok) return INF_ERR;
     const float dj = g.dj, u = g.u, v = g.v;
     if (!(dj > 0.f)) return INF_ERR;
-    f3 Yj = mk3((u - S.cx) / S.fx * dj, (v - S.cy) / S.fy * dj, dj);
+    f3 Yj;
+    if (S.plain) Yj = mk3(div_exact(u - S.cx, S.fx, S.ifx) * dj, div_exact(v - S.cy, S.fy, S.ify) * dj, dj);
+    else Yj = mk3((u - S.cx) / S.fx * dj, (v - S.cy) / S.fy * dj, dj);
     f3 q = mk3(Yj.x - pr.t[0], Yj.y - pr.t[1], Yj.z - pr.t[2]);
     float Yx = pr.r[0] * q.x + pr.r[3] * q.y + pr.r[6] * q.z;
     float Yy = pr.r[1] * q.x + pr.r[4] * q.y + pr.r[7] * q.z;
     float Yz = pr.r[2] * q.x + pr.r[5] * q.y + pr.r[8] * q.z;
     if (!(Yz > 1e-8f)) return INF_ERR;
-    float ex = R.fx * Yx / Yz + R.cx - (float)x, ey = R.fy * Yy / Yz + R.cy - (float)y;
+    float ex, ey;
+    if (Yz < EXACT_HI) {
+        const float iz = inv_exact(Yz);
+        ex = div_exact(R.fx * Yx, Yz, iz) + R.cx - (float)x;
+        ey = div_exact(R.fy * Yy, Yz, iz) + R.cy - (float)y;
+    } else {
+        ex = R.fx * Yx / Yz + R.cx - (float)x;
+        ey = R.fy * Yy / Yz + R.cy - (float)y;
+    }
     return sqrtf(ex * ex + ey * ey);
 }
 
@@ -811,7 +865,7 @@ __device__ __forceinline__ float pair_cost(const KParams& P, const RefWinT<WR, W
     float c = 2.0f;
     GeoFetch gf{0.f, 0.f, 0.f, false};
     if (P.geometric) gf = geo_fetch(P, R, S, pr, x, y, h.w);
-    if (homography(R, lp, 1.0f / R.fx, 1.0f / R.fy, (float)x, (float)y, h.w, xyz(h), H))
+    if (homography(R, lp, R.ifx, R.ify, (float)x, (float)y, h.w, xyz(h), H))
         c = ncc_cost_any<WR, WSTEP, PIPE>(P, rw, ref, S, H, x, y);
     if (P.geometric) *geo = fminf(geo_finish(R, S, pr, x, y, gf), P.gmax);
     return c;

@@ -188,7 +188,7 @@ void k_half(KParams P) {
     float4* pl = P.plane + base;
     const float* co = P.cost + base;
     const f3 ray = pixel_ray(R, x, y);
-    const float ifx = 1.0f / R.fx, ify = 1.0f / R.fy;
+    const float ifx = R.ifx, ify = R.ify;
     float* wv = wv_lds + threadIdx.x;
     float4* hyp = hyp_lds + threadIdx.x;  // hyp[i * NT]
 
@@ -259,36 +259,51 @@ void k_half(KParams P) {
         }
         wv[j * P.wv_stride] = 0.f;
         if (!(prior > 0.f)) continue;
-        float m[9], gg[9];
+        float m[9];  // photometric cost, then the term the aggregation takes: with lambda times the geometric error
+        int good = 0, bad = 0;
+        float conf = 0.f;
+        auto vote = [&](float mi) {
+            if (mi < P.tau_good) {
+                good++;
+                conf += c3d_expf(-mi * mi * P.inv2beta2);
+            }
+            if (mi > P.tau_bad) bad++;
+        };
 #pragma unroll
-        for (int q = 0; q < 9; ++q) m[q] = gg[q] = 0.f;
+        for (int q = 0; q < 9; ++q) m[q] = 0.f;
+        if constexpr (TPP == 1) {
 #pragma nounroll
-        for (int i = sub; i < 9; i += TPP) {
-            float gi;
-            const float mi = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lp, ifx, ify, x, y, hyp[i * NT], gi);
+            for (int i = 0; i < 9; ++i) {
+                float gi;
+                const float mi = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lp, ifx, ify, x, y, hyp[i * NT], gi);
+                if (i > 0) vote(mi);
+                const float ti = mi + P.lambda * gi;
 #pragma unroll
-            for (int q = 0; q < 9; ++q)
-                if (q == i) {
-                    m[q] = mi;
-                    gg[q] = gi;
-                }
-        }
-        if constexpr (TPP > 1) {
+                for (int q = 0; q < 9; ++q)
+                    if (q == i) m[q] = ti;
+            }
+        } else {
+            float gg[9];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) gg[q] = 0.f;
+#pragma nounroll
+            for (int i = sub; i < 9; i += TPP) {
+                float gi;
+                const float mi = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lp, ifx, ify, x, y, hyp[i * NT], gi);
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    if (q == i) {
+                        m[q] = mi;
+                        gg[q] = gi;
+                    }
+            }
 #pragma unroll
             for (int q = 0; q < 9; ++q) {
                 m[q] = __shfl(m[q], lane - sub + (q & (TPP - 1)));
                 if constexpr (GEO) gg[q] = __shfl(gg[q], lane - sub + (q & (TPP - 1)));
+                if (q > 0) vote(m[q]);
+                m[q] = m[q] + P.lambda * gg[q];
             }
-        }
-        int good = 0, bad = 0;
-        float conf = 0.f;
-#pragma unroll
-        for (int i = 1; i < 9; ++i) {
-            if (m[i] < P.tau_good) {
-                good++;
-                conf += c3d_expf(-m[i] * m[i] * P.inv2beta2);
-            }
-            if (m[i] > P.tau_bad) bad++;
         }
         bool adopt = good > P.n1 && bad < P.n2;
         bool isprev = j == vprev;
@@ -303,7 +318,7 @@ void k_half(KParams P) {
         if (adopted || !(den > 0.f)) {
             const float wa = adopted ? w2 : prior;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) agg[i] += wa * (m[i] + P.lambda * gg[i]);
+            for (int i = 0; i < 9; ++i) agg[i] += wa * m[i];
         }
         denf += prior;
         if (adopted) {
@@ -608,7 +623,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eval_waves<
             float cphi = dot3(Sv, xyz(h)) / ls;
             if (cphi <= 0.f) continue;
             float H[9];
-            if (!homography(R, lps[j], 1.0f / R.fx, 1.0f / R.fy, (float)x, (float)y, h.w, xyz(h), H)) continue;
+            if (!homography(R, lps[j], R.ifx, R.ify, (float)x, (float)y, h.w, xyz(h), H)) continue;
             const GeoFetch gf = geo_fetch(P, R, S, pr, x, y, h.w);  // used after the window
             float m = ncc_cost_any<WR, WSTEP, EVAL_PIPE>(P, rw, ref, S, H, x, y);
             float e = P.ncc_norm * c3d_expf(-m * m * P.inv2ncc);
@@ -638,7 +653,7 @@ __global__ __launch_bounds__(256) void k_pair_costs(KParams P, int view, int slo
     float4 h = planes[i];
     float H[9];
     float c = 2.f;
-    if (homography(R, lp, 1.0f / R.fx, 1.0f / R.fy, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP>(P, rw, g, S, H, x, y);
+    if (homography(R, lp, R.ifx, R.ify, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP>(P, rw, g, S, H, x, y);
     out[i] = c;
 }
 

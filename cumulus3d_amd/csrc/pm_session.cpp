@@ -603,6 +603,9 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
             L.fy = li.k[1];
             L.cx = li.k[2];
             L.cy = li.k[3];
+            L.ifx = 1.0f / L.fx;
+            L.ify = 1.0f / L.fy;
+            L.plain = std::fabs(L.fx) > 0x1p-20f && std::fabs(L.fx) < 0x1p40f && std::fabs(L.fy) > 0x1p-20f && std::fabs(L.fy) < 0x1p40f;
         }
     auto bail = [&](int code) {
         c3d_pm_end(s);
