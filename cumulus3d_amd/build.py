@@ -44,9 +44,13 @@ def _engine(name: str, defines: list[str]) -> str:
     os.makedirs(os.path.join(LIB, "obj"), exist_ok=True)
     objs = []
     jobs = []
-    for src in ("pm_kernels.hip", "pm_session.cpp", "nn_kernels.hip", "nn_net.cpp", "fusion.hip", "postproc.hip", "neighbors.hip"):
-        obj = os.path.join(LIB, "obj", f"{name}_{os.path.splitext(src)[0]}.o")
-        jobs.append([HIPCC, *HIP_FLAGS, *defines, "-c", os.path.join(CSRC, src), "-o", obj])
+    units = [(src, os.path.splitext(src)[0], []) for src in
+             ("pm_kernels.hip", "pm_session.cpp", "nn_kernels.hip", "nn_net.cpp", "fusion.hip", "postproc.hip", "neighbors.hip")]
+    # the window kernels, once for each form of the quad tables (the two longest compilations: first)
+    units[:0] = [("pm_windows.hip", f"pm_windows{b}", [f"-DC3D_QUAD_BYTES={b}"]) for b in (4, 8)]
+    for src, unit, extra in units:
+        obj = os.path.join(LIB, "obj", f"{name}_{unit}.o")
+        jobs.append([HIPCC, *HIP_FLAGS, *defines, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     with ThreadPoolExecutor(4) as ex:
         list(ex.map(_run, jobs))

@@ -2,11 +2,14 @@
 //
 // Layout in HBM (one session):
 //   gray   all view-level images, u8 row-major, no padding (reference patch loads)
-//   quad   per view-level, a (w+3) x (h+3) table of u32: entry (x0, y0) for x0 in [-2, w],
-//          y0 in [-2, h] packs the bilinear 2x2 neighbourhood p(x0,y0) | p(x0+1,y0) << 8 |
-//          p(x0,y0+1) << 16 | p(x0+1,y0+1) << 24 with 0 outside the image, so that one dword load
-//          gives all four texels of a source sample and clamping the integer sample position into
-//          the table reproduces "0 outside" exactly (patchmatch.cu:169-192 software bilinear).
+//   quad   per view-level, a (w+3) x (h+3) table: entry (x0, y0) for x0 in [-2, w], y0 in [-2, h] holds
+//          the bilinear 2x2 neighbourhood p(x0,y0), p(x0+1,y0), p(x0,y0+1), p(x0+1,y0+1) with 0 outside
+//          the image, so that one load gives all four texels of a source sample and clamping the
+//          integer sample position into the table reproduces "0 outside" exactly
+//          (patchmatch.cu:169-192 software bilinear). Two forms of the table, one per namespace of
+//          window kernels (pm_windows.hip is compiled for each): 4-byte entries of the four bytes, and
+//          8-byte entries of the row starts and row differences as half floats (exact), which save
+//          the four instructions that form them; which one a launch takes is run_quad8's rule.
 //   plane  float4 (nx, ny, nz, d) per pixel, row-major per view, views of a batch back to back
 //          (ViewState packed as in patchmatch.rs:327-348); cost f32, best view u8, count u8 alike.
 //
@@ -21,6 +24,10 @@
 
 #include <type_traits>
 
+#ifndef C3D_QUAD_BYTES
+#define C3D_QUAD_BYTES 4
+#endif
+
 namespace c3d {
 
 constexpr int MAXSRC = 32;
@@ -31,7 +38,7 @@ struct LevelDesc {
     int w, h;
     int qpitch;      // quad row pitch (w + 3)
     int pad0;
-    long long qoff;  // dword offset of quad entry (0, 0) (the 2-texel border precedes it)
+    long long qoff;  // index of quad entry (0, 0) (the 2-texel border precedes it)
     long long goff;  // byte offset of the u8 image
     float fx, fy, cx, cy;
     float ifx, ify;   // 1 / fx, 1 / fy
@@ -63,7 +70,7 @@ struct BatchItem {
 struct KParams {
     unsigned long long seed;
     const uint8_t* gray;
-    const uint32_t* quad;
+    const void* quad;  // entries of 4 or 8 bytes: the table of the launched kernels' namespace
     const LevelDesc* lv;
     const PairRec* pairs;
     const LevelPair* lpairs;
@@ -158,6 +165,47 @@ __device__ __forceinline__ bool locate_tile_pre(const KParams& P, int t, int tw,
 __device__ __forceinline__ bool find_tile(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0) {
     return P.tile_pre ? locate_tile_pre(P, t, tw, th, it, x0, y0) : locate_tile(P, t, tw, th, it, x0, y0);
 }
+
+// ---------------------------------------------------------------- tile shapes
+
+// Waves per half-step workgroup ("rows": one row of blocks each): a compile-time variant (1, 2 or
+// 4), picked per session by the tile autotuner (c3d_pm_autotune). One is the default: a wave's slot
+// on its SIMD is refilled as soon as that wave ends, where a 4-wave workgroup holds its slots (and
+// its LDS) until its slowest wave is done, and the waves' work differs through the data-dependent
+// early exits.
+constexpr int HALF_SPAN = 128;   // pixel span of one row of 64 active pixels (k_eval of one colour)
+// A wave of the half step takes a block of half_bw x half_bh pixels, half of them active: 16 x 8, or
+// 8 x 8, 8 x 4 and 8 x 2 with two, four and eight lanes per pixel. What
+// a wave costs is what its costliest lane costs, window by window, and pixels of a compact block
+// agree better on it (which sources see them, when a candidate is given up) than 64 pixels along
+// 128 of one row: 3.4 % fewer VALU instructions for the same pixels. The block's samples also share
+// more source lines (a third of the L1 misses of the row), a ragged width wastes less, and the
+// staged tile is 2.9 instead of 6.1 KB. 9 views of 1920 x 1080 with 6 sources: half step
+// 23.5 -> 22.2 ms; 2 such views, 3 iterations from a random start: 35.3 -> 31.9 ms; one of
+// 160 x 96: 0.69 -> 0.61 ms.
+__host__ __device__ constexpr int half_bw(int tpp) { return tpp == 1 ? 16 : 8; }
+__host__ __device__ constexpr int half_bh(int tpp) { return tpp <= 2 ? 8 : 16 / tpp; }
+
+// Active pixel p of a wave's block as (column of active pixels, row): four neighbouring lanes take a
+// 2 x 2 group, so that lanes next to each other sample next to each other in the source, whichever
+// way it is turned against the reference.
+template <int TPP>
+__device__ __forceinline__ void block_pixel(int p, int& col, int& row) {
+    col = (p & 1) | ((p >> 1) & 2);
+    row = (p >> 1) & 1;
+    if (TPP == 1) {
+        col |= (p >> 2) & 4;
+        row |= ((p >> 2) & 2) | ((p >> 3) & 4);
+    } else {
+        row |= (p >> 2) & 6;
+    }
+}
+
+// Pitch of the staged reference rows: the block with its margins, rounded up to 8 modulo 16, with
+// which the 64 lanes of a block read 64 different LDS banks.
+__host__ __device__ constexpr int half_pitch(int tpp, int wr) { return ((half_bw(tpp) + 2 * wr + 7) / 16) * 16 + 8; }
+constexpr int PIX_TW = 64;       // eval/filter tiles: 64 x 4 pixels
+constexpr int PIX_TH = 4;
 
 // ---------------------------------------------------------------- random numbers (kernel.rs:248-259)
 
@@ -401,41 +449,70 @@ __device__ __forceinline__ bool homography(const LevelDesc& R, const LevelPair& 
     return true;
 }
 
-// Bilinear interpolation of one quad entry q = p00 | p10 << 8 | p01 << 16 | p11 << 24 at the
-// fractions (ax, ay): top = p00 + ax (p10 - p00), bot = p01 + ax (p11 - p01), top + ay (bot - top),
-// each an FP32 FMA. The two row starts and the two row differences are formed as packed half
-// floats: a byte permute sets the exponent byte 0x64 above each texel, which reads 1024 + p
-// exactly, and one packed subtraction each gives (p00, p01) and (p10 - p00, p11 - p01), all
-// integers of magnitude below 2^11 and so exact. Each row is then one mixed FMA on the exact
-// half-float operands: the same value as the FP32 formula, in 8 instructions instead of 10.
+// Bilinear interpolation of one quad entry at the fractions (ax, ay): top = p00 + ax (p10 - p00),
+// bot = p01 + ax (p11 - p01), top + ay (bot - top), each an FP32 FMA. The two row starts and the two
+// row differences are packed half floats (integers of magnitude below 2^11, exact), and each row is
+// one mixed FMA on them: the same value as the FP32 formula. From a 4-byte entry p00 | p10 << 8 |
+// p01 << 16 | p11 << 24 they take a byte permute each that sets the exponent byte 0x64 above each
+// texel, which reads 1024 + p exactly, and a packed subtraction each; an 8-byte entry holds them.
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t quad_lo(uint32_t q) { return __builtin_amdgcn_perm(0x64646464u, q, 0x04020400u); }  // (1024 + p00, 1024 + p01)
-__device__ __forceinline__ uint32_t quad_hi(uint32_t q) { return __builtin_amdgcn_perm(0x64646464u, q, 0x04030401u); }  // (1024 + p10, 1024 + p11)
-__device__ __forceinline__ float quad_lerp(uint32_t q, float ax, float ay) {
-    const half2_t l = __builtin_bit_cast(half2_t, quad_lo(q)), h = __builtin_bit_cast(half2_t, quad_hi(q));
-    const half2_t d = h - l;
-    const half2_t p = l - (half2_t){(_Float16)1024.0f, (_Float16)1024.0f};
+__device__ __forceinline__ uint32_t quad_entry4(uint32_t p00, uint32_t p10, uint32_t p01, uint32_t p11) {
+    return p00 | (p10 << 8) | (p01 << 16) | (p11 << 24);
+}
+__device__ __forceinline__ uint2 quad_entry8(uint32_t p00, uint32_t p10, uint32_t p01, uint32_t p11) {
+    const half2_t p = {(_Float16)(int)p00, (_Float16)(int)p01};
+    const half2_t d = {(_Float16)((int)p10 - (int)p00), (_Float16)((int)p11 - (int)p01)};
+    return make_uint2(__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, d));
+}
+#if C3D_QUAD_BYTES == 8
+typedef uint2 QuadEntry;
+__device__ __forceinline__ void quad_rows(QuadEntry q, half2_t& p, half2_t& d) {
+    p = __builtin_bit_cast(half2_t, q.x);
+    d = __builtin_bit_cast(half2_t, q.y);
+}
+#else
+typedef uint32_t QuadEntry;
+__device__ __forceinline__ void quad_rows(QuadEntry q, half2_t& p, half2_t& d) {
+    const half2_t l = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, q, 0x04020400u));  // (1024 + p00, 1024 + p01)
+    const half2_t h = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, q, 0x04030401u));  // (1024 + p10, 1024 + p11)
+    d = h - l;
+    p = l - (half2_t){(_Float16)1024.0f, (_Float16)1024.0f};
+}
+#endif
+__device__ __forceinline__ float quad_lerp(QuadEntry q, float ax, float ay) {
+    half2_t p, d;
+    quad_rows(q, p, d);
     const float top = fmaf(ax, (float)d.x, (float)p.x);
     const float bot = fmaf(ax, (float)d.y, (float)p.y);
     return fmaf(ay, bot - top, top);
 }
 
-// One source sample in gray levels through the quad table (see the layout note above). `qbase` is
-// the table's first entry (x0, y0) = (-2, -2); the byte offset 4 ((y0 + 2) qpitch + (x0 + 2)) is formed
-// exactly in FP32 (multiples of 4 below 2^26) from the clamped floor of the sample position, and the
-// load uses a uniform base plus a 32-bit offset.
-__device__ __forceinline__ uint32_t quad_fetch(const uint32_t* qbase, float qp4, float koff4, float w1, float h1, float u, float v,
-                                               float& ax, float& ay) {
+// The quad table of a source as the samples use it: `base` is the table's first entry (x0, y0) =
+// (-2, -2); the byte offset of an entry, QB ((y0 + 2) qpitch + (x0 + 2)), is formed exactly in FP32
+// (multiples of QB below 2^24 QB) from the clamped floor of the sample position, and the load uses
+// the uniform base plus a 32-bit offset.
+constexpr float QB = (float)sizeof(QuadEntry);
+struct QuadTable {
+    const QuadEntry* base;
+    float pitch, off, w, h;
+};
+__device__ __forceinline__ QuadTable quad_table(const KParams& P, const LevelDesc& S) {
+    const float pitch = QB * (float)S.qpitch;
+    return QuadTable{(const QuadEntry*)P.quad + (S.qoff - 2LL * S.qpitch - 2), pitch, 2.0f * pitch + 2.0f * QB, (float)S.w, (float)S.h};
+}
+__device__ __forceinline__ QuadEntry quad_load(const QuadTable& t, float xc, float yc) {
+    return *(const QuadEntry*)((const char*)t.base + (uint32_t)fmaf(yc, t.pitch, fmaf(xc, QB, t.off)));
+}
+// one source sample in gray levels: the entry and the fractions
+__device__ __forceinline__ QuadEntry quad_fetch(const QuadTable& t, float u, float v, float& ax, float& ay) {
     const float xf = floorf(u), yf = floorf(v);
     ax = u - xf;
     ay = v - yf;
-    const float xc = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
-    const float yc = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
-    return *(const uint32_t*)((const char*)qbase + (uint32_t)fmaf(yc, qp4, fmaf(xc, 4.0f, koff4)));
+    return quad_load(t, __builtin_amdgcn_fmed3f(xf, -2.0f, t.w), __builtin_amdgcn_fmed3f(yf, -2.0f, t.h));
 }
-__device__ __forceinline__ float quad_sample(const uint32_t* qbase, float qp4, float koff4, float w1, float h1, float u, float v) {
+__device__ __forceinline__ float quad_sample(const QuadTable& t, float u, float v) {
     float ax, ay;
-    const uint32_t q = quad_fetch(qbase, qp4, koff4, w1, h1, u, v, ax, ay);
+    const QuadEntry q = quad_fetch(t, u, v, ax, ay);
     return quad_lerp(q, ax, ay);
 }
 
@@ -457,8 +534,8 @@ constexpr int WINDOW_PIPE = 8;
 // LDS per sample; it fits their registers); the evaluation and read-out, held to three waves
 // per SIMD, would spill with it.
 template <int WR, int WSTEP, bool CHECK, int PIPE, bool AHEAD, class REF>
-__device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y, const uint32_t* qbase, float qp4,
-                                            float koff4, float w1, float h1, const float* H, float& Ss, float& SSs, float& IS) {
+__device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y, const QuadTable& qt,
+                                            const float* H, float& Ss, float& SSs, float& IS) {
     constexpr int WN = Win<WR, WSTEP>::WN;
     constexpr int N = WN * WN;
     Ss = 0.f;
@@ -468,7 +545,7 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
     // sample k is used up, so PIPE gathers stay in flight. The sums take the samples in row-major
     // order.
     float fx[N], fy[N], rv[N];
-    uint32_t qv[N];
+    QuadEntry qv[N];
     float rz = 0.f, ru = 0.f, rt = 0.f;  // the issued row's projective terms at dx = 0
     auto xoff = [](int k) { return -WR + (k % WN) * WSTEP; };
     auto yoff = [](int k) { return -WR + (k / WN) * WSTEP; };
@@ -483,7 +560,7 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
         if constexpr (AHEAD) rv[k] = ref.at(x + xoff(k), y + yoff(k));
         const float ox = (float)xoff(k);
         const float r = rcp_sample(fmaf(H[6], ox, rz));
-        qv[k] = quad_fetch(qbase, qp4, koff4, w1, h1, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rt) * r, fx[k], fy[k]);
+        qv[k] = quad_fetch(qt, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rt) * r, fx[k], fy[k]);
     };
 #pragma unroll
     for (int k = 0; k < PIPE && k < N; ++k) issue(k);
@@ -500,15 +577,16 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
             if constexpr (AHEAD) rv[n] = ref.at(x + xoff(n), y + yoff(n));
             zz = fmaf(H[6], (float)xoff(n), rz);
         }
-        const uint32_t lo = quad_lo(qv[k]);
-        if (more) r = rcp_seed(zz);
-        const uint32_t hi = quad_hi(qv[k]);
-        if (more) e = fmaf(-zz, r, 1.0f);
-        const half2_t l = __builtin_bit_cast(half2_t, lo);
-        const half2_t d = __builtin_bit_cast(half2_t, hi) - l;
-        if (more) e = fmaf(e, e, e);
-        const half2_t p = l - (half2_t){(_Float16)1024.0f, (_Float16)1024.0f};
-        if (more) r = fmaf(r, e, r);
+        if (more) {
+            r = rcp_seed(zz);
+            e = fmaf(-zz, r, 1.0f);
+        }
+        half2_t p, d;
+        quad_rows(qv[k], p, d);
+        if (more) {
+            e = fmaf(e, e, e);
+            r = fmaf(r, e, r);
+        }
         const float top = fmaf(fx[k], (float)d.x, (float)p.x);
         if (more) e = fmaf(-zz, r, 1.0f);
         const float bot = fmaf(fx[k], (float)d.y, (float)p.y);
@@ -531,11 +609,10 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
         if (more) fx[n] = u - xf;
         IS = fmaf(ws, AHEAD ? rv[k] : ref.at(x + xoff(k), y + yoff(k)), IS);
         if (more) {
-            xf = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
+            xf = __builtin_amdgcn_fmed3f(xf, -2.0f, qt.w);
             fy[n] = v - yf;
-            yf = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
-            xf = fmaf(xf, 4.0f, koff4);
-            qv[n] = *(const uint32_t*)((const char*)qbase + (uint32_t)fmaf(yf, qp4, xf));
+            yf = __builtin_amdgcn_fmed3f(yf, -2.0f, qt.h);
+            qv[n] = quad_load(qt, xf, yf);
         }
     }
 }
@@ -549,7 +626,7 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
 // 3 % slower on 9 views of 1920 x 1080 (spills).
 template <int WR, int WSTEP, class REF>
 __device__ __forceinline__ void window_sums_behind(const KParams& P, const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y,
-                                                   const uint32_t* qbase, float qp4, float koff4, float w1, float h1, const float* H,
+                                                   const QuadTable& qt, const float* H,
                                                    float& Ss, float& SSs, float& IS) {
     constexpr int WN = Win<WR, WSTEP>::WN;
     constexpr int CH = 3;
@@ -564,13 +641,13 @@ __device__ __forceinline__ void window_sums_behind(const KParams& P, const RefWi
 #pragma unroll 1
         for (int b0 = 0; b0 < WN; b0 += CH) {
             float fx[CH], fy[CH], zs[CH];
-            uint32_t qv[CH];
+            QuadEntry qv[CH];
 #pragma unroll
             for (int g = 0; g < CH; ++g) {
                 const float ox = (float)(-WR + (b0 + g) * WSTEP);
                 zs[g] = fmaf(H[6], ox, rz);
                 const float r = rcp_sample(zs[g]);
-                qv[g] = quad_fetch(qbase, qp4, koff4, w1, h1, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r, fx[g], fy[g]);
+                qv[g] = quad_fetch(qt, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r, fx[g], fy[g]);
             }
 #pragma unroll
             for (int g = 0; g < CH; ++g) {
@@ -603,20 +680,18 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
     // inside the source (a NaN position is not)
     if (!(__builtin_amdgcn_fmed3f(u, 0.f, (float)(S.w - 1)) == u && __builtin_amdgcn_fmed3f(v, 0.f, (float)(S.h - 1)) == v)) return 2.0f;
     if (rw.var < P.vmin255) return 2.0f;
-    const uint32_t* qbase = P.quad + (S.qoff - 2LL * S.qpitch - 2);
-    const float qp4 = 4.0f * (float)S.qpitch, koff4 = 2.0f * qp4 + 8.0f;
-    const float w1 = (float)S.w, h1 = (float)S.h;
+    const QuadTable qt = quad_table(P, S);
     constexpr float lo = (float)(-WR), hi = (float)Win<WR, WSTEP>::LAST;
     const float za = fmaf(H[7], lo, H[8]), zb = fmaf(H[7], hi, H[8]);
     const bool all_front = fmaf(H[6], lo, za) > 1e-8f && fmaf(H[6], hi, za) > 1e-8f && fmaf(H[6], lo, zb) > 1e-8f &&
                            fmaf(H[6], hi, zb) > 1e-8f;
     float Ss, SSs, IS;
     if (all_front) {
-        window_sums<WR, WSTEP, false, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+        window_sums<WR, WSTEP, false, PIPE, AHEAD>(rw, ref, x, y, qt, H, Ss, SSs, IS);
     } else if constexpr (COPY) {
-        window_sums<WR, WSTEP, true, PIPE, AHEAD>(rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+        window_sums<WR, WSTEP, true, PIPE, AHEAD>(rw, ref, x, y, qt, H, Ss, SSs, IS);
     } else {
-        window_sums_behind<WR, WSTEP>(P, rw, ref, x, y, qbase, qp4, koff4, w1, h1, H, Ss, SSs, IS);
+        window_sums_behind<WR, WSTEP>(P, rw, ref, x, y, qt, H, Ss, SSs, IS);
     }
     const float iW = rw.iW;
     float mus = Ss * iW;
@@ -695,9 +770,7 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
     // inside the source (a NaN position is not)
     if (!(__builtin_amdgcn_fmed3f(u, 0.f, (float)(S.w - 1)) == u && __builtin_amdgcn_fmed3f(v, 0.f, (float)(S.h - 1)) == v)) return 2.0f;
     if (rw.var < P.vmin255) return 2.0f;
-    const uint32_t* qbase = P.quad + (S.qoff - 2LL * S.qpitch - 2);
-    const float qp4 = 4.0f * (float)S.qpitch, koff4 = 2.0f * qp4 + 8.0f;
-    const float w1 = (float)S.w, h1 = (float)S.h;
+    const QuadTable qt = quad_table(P, S);
     const int wr = rw.wr, wn = (2 * wr) / WSTEP + 1;
     float Ss = 0.f, SSs = 0.f, IS = 0.f;
     for (int a = 0; a < wn; ++a) {
@@ -713,7 +786,7 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
                 const float ox = (float)dxi;
                 const float zz = fmaf(H[6], ox, rz);
                 const float r = rcp_sample(zz);
-                float sv = quad_sample(qbase, qp4, koff4, w1, h1, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r);
+                float sv = quad_sample(qt, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r);
                 sv = zz > 1e-8f ? sv : 0.0f;
                 const float iv = ref.at(x + dxi, y + dyi);
                 const float sp = sv - rw.ic;
@@ -728,7 +801,7 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
         // samples past the row's end in the last chunk repeat its last sample and are not summed);
         // faster in the geometric builds, slower in the photometric one
         for (int b0 = 0; b0 < wn; b0 += 4) {
-            uint32_t qs[4];
+            QuadEntry qs[4];
             float fxs[4], fys[4], zs[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -737,20 +810,15 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
                 const float zz = fmaf(H[6], ox, rz);
                 const float r = rcp_sample(zz);
                 const float su = fmaf(H[0], ox, ru) * r, sw = fmaf(H[3], ox, rv) * r;
-                const float xf = floorf(su), yf = floorf(sw);
-                fxs[u] = su - xf;
-                fys[u] = sw - yf;
                 zs[u] = zz;
-                const float xc = __builtin_amdgcn_fmed3f(xf, -2.0f, w1);
-                const float yc = __builtin_amdgcn_fmed3f(yf, -2.0f, h1);
-                qs[u] = *(const uint32_t*)((const char*)qbase + (uint32_t)fmaf(yc, qp4, fmaf(xc, 4.0f, koff4)));
+                qs[u] = quad_fetch(qt, su, sw, fxs[u], fys[u]);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int b = b0 + u;
                 if (b >= wn) break;
                 const int dxi = -wr + b * WSTEP;
-                const uint32_t q = qs[u];
+                const QuadEntry q = qs[u];
                 const float ax = fxs[u], ay = fys[u];
                 float sv = quad_lerp(q, ax, ay);
                 sv = zs[u] > 1e-8f ? sv : 0.0f;
@@ -951,6 +1019,23 @@ __device__ __forceinline__ float view_prior(const KParams& P, const LevelDesc& R
     if (!(area > 0.f)) return 0.f;
     float res = fminf(area / aref, aref / area);
     return tri * inc * res;
+}
+
+// ---------------------------------------------------------------- run start
+
+// The plane a run starts from (mode 1: initialised where random_init says so, patchmatch.cu:668-677).
+__device__ __forceinline__ float4 eval_init_plane(const KParams& P, const ViewDesc& vd, const LevelDesc& R, int x, int y, int pix,
+                                                  long long base, int mode) {
+    float4 h = P.plane[base + pix];
+    // random_init 1: every pixel (patchmatch.cu:668-676); 2: pixels without a positive depth
+    if (mode == 1 && (P.random_init == 1 || (P.random_init == 2 && !(h.w > 0.f)))) {
+        unsigned long long st = rng_state(P.seed, vd.key, P.level, P.run_id, 0xFFFF, 0, (unsigned long long)pix);
+        float d = random_depth(st, vd.dmin, vd.dmax);
+        f3 n = random_normal(st, pixel_ray(R, x, y));
+        h = mk4(n, d);
+        P.plane[base + pix] = h;
+    }
+    return h;
 }
 
 }  // namespace c3d

@@ -21,7 +21,8 @@ struct KernelSet {
 // Kernels of a window (radius 1..MAX_WR, step 1 or 2): the fixed-radius build when compiled and
 // `any_radius` is false, else the any-radius kernels of the step (KernelSet::wr == 0); nullptr
 // outside those bounds.
-const KernelSet* kernel_set(int wr, int wstep, bool any_radius);
+// quad_bytes: the kernels that sample tables of 4-byte or of 8-byte quad entries.
+const KernelSet* kernel_set(int wr, int wstep, bool any_radius, int quad_bytes);
 
 // half-step workgroup shapes compiled: (rows of a workgroup, lanes per pixel) = (1, 1), (2, 1), (4, 1), (4, 2)
 bool half_shape_ok(int rows, int tpp);
@@ -40,7 +41,7 @@ hipError_t launch_split_planes(const float4* plane, float* depth, float* normal,
 hipError_t launch_merge_planes(const float* depth, const float* normal, float4* plane, long long n, hipStream_t s);
 hipError_t launch_upsample(const KParams& P, hipStream_t s);
 hipError_t launch_median(const KParams& P, hipStream_t s);
-hipError_t launch_quad_build(const uint8_t* g, int w, int h, uint32_t* q, hipStream_t s);
+hipError_t launch_quad_build(const uint8_t* g, int w, int h, uint32_t* q4, uint2* q8, hipStream_t s);
 hipError_t launch_extract_depth(const float4* plane, float* out, long long n, hipStream_t s);
 hipError_t launch_restore(float4* plane, const float4* up, const float* c_init, float* cost, float xi, long long n,
                           hipStream_t s);
@@ -49,5 +50,13 @@ hipError_t launch_threshold(const KParams& P, const uint8_t* need, float4* out, 
 hipError_t launch_half_tile_prefix(const BatchItem* batch, int n, int rows, int tpp, int* pre, hipStream_t s);
 hipError_t launch_pix_tile_prefix(const BatchItem* batch, int n, int* pre, hipStream_t s);
 hipError_t launch_span_tile_prefix(const BatchItem* batch, int n, int* pre, hipStream_t s);
+
+// the two builds of pm_windows.hip
+namespace quad4 {
+const KernelSet* kernel_set(int wr, int wstep, bool any_radius);
+}  // namespace quad4
+namespace quad8 {
+const KernelSet* kernel_set(int wr, int wstep, bool any_radius);
+}  // namespace quad8
 
 }  // namespace c3d

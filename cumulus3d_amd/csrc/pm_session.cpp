@@ -157,10 +157,13 @@ void backend_release(c3d_pm_backend* be) {
 }
 }  // namespace c3d
 
+// Sessions of more quad entries (view-level pixels) keep the 4-byte table only: the second one is at most 4 GiB.
+constexpr size_t QUAD8_ENTRIES = (size_t)1 << 29;
+
 struct c3d_pm_session {
     c3d_pm_backend* be = nullptr;
     std::unique_lock<std::mutex> guard;
-    const KernelSet* ks = nullptr;
+    const KernelSet* ks[2] = {};  // window kernels for quad entries of 4 and of 8 bytes
     int nv = 0, nl = 0;
     std::vector<LevelDesc> lv;
     std::vector<ViewDesc> vd;
@@ -169,6 +172,7 @@ struct c3d_pm_session {
     // device tables
     DevBuf<uint8_t> gray;
     DevBuf<uint32_t> quad;
+    DevBuf<uint2> quad8;  // none in sessions of more than QUAD8_ENTRIES
     DevBuf<LevelDesc> d_lv;
     DevBuf<PairRec> d_pairs;
     DevBuf<LevelPair> d_lpairs;
@@ -296,10 +300,17 @@ int set_batch(c3d_pm_session* s, const uint32_t* views, uint32_t a, uint32_t b, 
     return C3D_OK;
 }
 
+// The window kernels of a launch and, in k, the quad table that they sample (run_quad8's rule for
+// a run; wide for planes that are given).
+const KernelSet* use_quads(const c3d_pm_session* s, KParams& k, bool wide) {
+    wide = wide && s->quad8.p;
+    k.quad = wide ? (const void*)s->quad8.p : (const void*)s->quad.p;
+    return s->ks[wide];
+}
+
 KParams params_for(c3d_pm_session* s, uint32_t level, bool geometric, const std::vector<BatchItem>& items, int max_nsrc) {
     KParams k = s->base;
     k.gray = s->gray.p;
-    k.quad = s->quad.p;
     k.lv = s->d_lv.p;
     k.pairs = s->d_pairs.p;
     k.lpairs = s->d_lpairs.p;
@@ -380,17 +391,38 @@ void iteration_constants(const c3d_pm_params& pm, bool geometric, uint32_t t, KP
     k.phi = deg2rad(std::fmax(phi0 * p, pm.phi_min_deg));
 }
 
+// Which of the two quad tables a run takes. The 8-byte entries save 4 of a sample's 33 instructions and
+// double what the samples touch. Where neighbouring pixels sample near each other that pays: half
+// step of 9 views of 1920 x 1080 with 6 sources from the network's planes 19.3 -> 17.9 ms, 24
+// geometric views of 480 x 270 25.7 -> 24.7 ms a run, evaluation and read-out filter of the 9 views
+// 3.07 -> 2.75 ms. A run from random planes samples all over its sources, waits for L2 misses, and
+// loses unless the tables are small, first iteration and later ones (6 views, 6 sources, 4-byte and
+// 8-byte): 1920 x 1080 43.1 and 54.1, 24.6 and 25.3 ms; 960 x 540 9.9 and 12.0, 6.41 and 6.15 ms;
+// 480 x 270 (12 views) 5.9 and 5.9, 4.1 and 3.7 ms.
+constexpr long long RANDOM_QUAD8 = 1 << 18;        // largest source image of a random run for 8-byte entries throughout
+constexpr long long RANDOM_QUAD8_LATER = 1 << 20;  // and for 8-byte entries after the first iteration
+bool run_quad8(const c3d_pm_session* s, const KParams& k, const std::vector<BatchItem>& items, uint32_t t) {
+    if (k.random_init != 1) return true;
+    for (const BatchItem& it : items)
+        for (int j = 0; j < s->vd[it.view].nsrc; ++j) {
+            const LevelDesc& S = s->lv[(size_t)s->h_pair_src[(size_t)it.view * MAXSRC + j] * s->nl + k.level];
+            if ((long long)S.w * S.h > (t == 0 ? RANDOM_QUAD8 : RANDOM_QUAD8_LATER)) return false;
+        }
+    return true;
+}
+
 // One run over the current batch: eval mode 1, then iterations x colours (patchmatch.rs:766-779).
 // With `timed`, every half-step launch is bracketed by a pair of pool events (read later).
 int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items, const c3d_pm_params& pm, bool geometric,
                uint32_t iterations, bool timed) {
     hipStream_t st = s->be->stream;
+    const KernelSet* ks = use_quads(s, k, run_quad8(s, k, items, 0));
     k.ntiles = pix_tiles(items.data(), (int)items.size());
     if (iterations == 0) {
         HIP_TRY(launch_pix_tile_prefix(k.batch, k.nitems, s->tile_pre.p, st));
         KParams e = k;
         e.tile_pre = s->tile_pre.p;
-        HIP_TRY(s->ks->eval(e, 1, st));
+        HIP_TRY(ks->eval(e, 1, st));
     } else {
         // the colour-0 costs of the run start are overwritten unread by the first half step: only
         // colour 1 is costed (k_eval_init initialises every pixel and resets the best view)
@@ -401,7 +433,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
         e.ntiles = span_tiles(items.data(), (int)items.size());
         HIP_TRY(launch_span_tile_prefix(e.batch, e.nitems, s->tile_pre.p, st));
         e.tile_pre = s->tile_pre.p;
-        HIP_TRY(s->ks->eval_color(e, st));
+        HIP_TRY(ks->eval_color(e, st));
     }
     const int tpp = s->half_auto ? half_lanes(items.data(), (int)items.size()) : s->half_tpp;
     k.ntiles = half_tiles(items.data(), (int)items.size(), s->half_rows, tpp);
@@ -411,6 +443,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
     }
     for (uint32_t t = 0; t < iterations; ++t) {
         iteration_constants(pm, geometric, t, k);
+        if (t == 1) ks = use_quads(s, k, run_quad8(s, k, items, t));
         for (int color = 0; color < 2; ++color) {
             k.color = color;
             if (timed) {
@@ -421,7 +454,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
                 }
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used], st));
             }
-            HIP_TRY(s->ks->half(k, s->half_rows, tpp, st));
+            HIP_TRY(ks->half(k, s->half_rows, tpp, st));
             if (timed) {
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used + 1], st));
                 s->pool_used += 2;
@@ -540,8 +573,9 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     if (pm.window_radius < 1 || pm.window_radius > 20 || pm.window_step < 1 || pm.window_step > 2)
         return fail(C3D_INVALID_ARGUMENT, "window radius " + std::to_string(pm.window_radius) + " (1..=20), step " +
                                               std::to_string(pm.window_step) + " (1|2)");
-    const KernelSet* ks = kernel_set(pm.window_radius, pm.window_step, be->opts.any_radius != 0);
-    if (!ks)
+    const KernelSet* ks = kernel_set(pm.window_radius, pm.window_step, be->opts.any_radius != 0, 4);
+    const KernelSet* ks8 = kernel_set(pm.window_radius, pm.window_step, be->opts.any_radius != 0, 8);
+    if (!ks || !ks8)
         return fail(C3D_INVALID_ARGUMENT, "window radius " + std::to_string(pm.window_radius) + " step " + std::to_string(pm.window_step) +
                                               " has no compiled kernels in this build");
     if (in->num_levels < 1) return fail(C3D_INVALID_ARGUMENT, "num_levels must be >= 1");
@@ -579,7 +613,8 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     c3d_pm_session* s = new c3d_pm_session();
     s->be = be;
     hold.kept = true;  // the session owns the hold from here; c3d_pm_end gives it back
-    s->ks = ks;
+    s->ks[0] = ks;
+    s->ks[1] = ks8;
     s->nv = nv;
     s->nl = nl;
     s->lv.resize((size_t)nv * nl);
@@ -617,14 +652,17 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     hipStream_t st = be->stream;
     if (s->gray.reserve(gtot) != hipSuccess || s->quad.reserve(qtot) != hipSuccess)
         return bail(fail(C3D_DEVICE, "HIP: out of device memory for images"));
+    // without room for the second table every launch takes the first
+    if (qtot <= QUAD8_ENTRIES && s->quad8.reserve(qtot) != hipSuccess) (void)hipGetLastError();
     for (int v = 0; v < nv; ++v)
         for (int l = 0; l < nl; ++l) {
             const c3d_level_image& li = in->views[v].levels[l];
             const LevelDesc& L = s->lv[(size_t)v * nl + l];
             if (hipMemcpyAsync(s->gray.p + L.goff, li.gray, (size_t)L.w * L.h, hipMemcpyHostToDevice, st) != hipSuccess)
                 return bail(fail(C3D_DEVICE, "HIP: image upload"));
-            if (launch_quad_build(s->gray.p + L.goff, L.w, L.h, s->quad.p + (L.qoff - 2LL * L.qpitch - 2), st) != hipSuccess)
-                return bail(fail(C3D_DEVICE, "HIP: quad build"));
+            const size_t q0 = (size_t)(L.qoff - 2LL * L.qpitch - 2);
+            if (launch_quad_build(s->gray.p + L.goff, L.w, L.h, s->quad.p + q0, s->quad8.p ? s->quad8.p + q0 : nullptr, st) != hipSuccess)
+                return bail(fail(C3D_DEVICE, "HIP: quad tables"));
         }
     std::vector<PairRec> prs((size_t)nv * MAXSRC);
     std::vector<LevelPair> lps((size_t)nv * nl * MAXSRC);
@@ -705,6 +743,7 @@ void c3d_pm_end(c3d_pm_session* s) {
     (void)hipStreamSynchronize(s->be->stream);
     s->gray.release();
     s->quad.release();
+    s->quad8.release();
     s->d_lv.release();
     s->d_pairs.release();
     s->d_lpairs.release();
@@ -805,7 +844,7 @@ int c3d_pm_evaluate(c3d_pm_session* s, uint32_t level, const uint32_t* views, ui
         if (rc) return rc;
         KParams k = params_for(s, level, geometric != 0, items, max_nsrc);
         k.ntiles = pix_tiles(items.data(), (int)items.size());
-        HIP_TRY(s->ks->eval(k, 0, st));
+        HIP_TRY(use_quads(s, k, true)->eval(k, 0, st));
         std::vector<c3d::Download> xs;
         for (size_t i = 0; i < items.size(); ++i)
             xs.push_back({(const unsigned char*)(s->cost.p + items[i].off), (unsigned char*)costs[a + i],
@@ -837,7 +876,7 @@ int c3d_pm_filter(c3d_pm_session* s, const uint32_t* views, uint32_t n, const c3
         if (rc) return rc;
         KParams k = params_for(s, level, true, items, max_nsrc);
         k.ntiles = pix_tiles(items.data(), (int)items.size());
-        HIP_TRY(s->ks->filter(k, st));
+        HIP_TRY(use_quads(s, k, true)->filter(k, st));
         std::vector<c3d::Download> xs;
         for (size_t i = 0; i < items.size(); ++i)
             xs.push_back({s->count.p + items[i].off, counts[a + i], (size_t)items[i].w * items[i].h});
@@ -1042,7 +1081,7 @@ int enqueue_densify(c3d_pm_session* s, const DensifyPlan& pl, const c3d_schedule
             KParams e = plan_params(s, pl, level, false);
             e.ntiles = pix_tiles(items, (int)pl.n);
             e.tile_pre = s->tile_pre.p;  // the 64 x 4 table built for the upsampling
-            HIP_TRY(s->ks->eval(e, 0, st));
+            HIP_TRY(use_quads(s, e, true)->eval(e, 0, st));
             HIP_TRY(hipMemcpyAsync(s->cinit.p, s->cost.p, (size_t)npix * sizeof(float), hipMemcpyDeviceToDevice, st));
             KParams k = plan_params(s, pl, level, false);
             k.run_id = (int)run_id++;
@@ -1051,7 +1090,7 @@ int enqueue_densify(c3d_pm_session* s, const DensifyPlan& pl, const c3d_schedule
             int rc = launch_run(s, k, iv, s->pm_copy, false, sch->photometric_iters_upper, timed);
             if (rc) return rc;
             HIP_TRY(launch_pix_tile_prefix(e.batch, e.nitems, s->tile_pre.p, st));  // the run rebuilt it
-            HIP_TRY(s->ks->eval(e, 0, st));
+            HIP_TRY(use_quads(s, e, true)->eval(e, 0, st));
             HIP_TRY(launch_restore(s->plane.p, s->up.p, s->cinit.p, s->cost.p, sch->restorer_threshold, npix, st));
         }
         if (timed) MARK(1);
@@ -1082,7 +1121,7 @@ int enqueue_densify(c3d_pm_session* s, const DensifyPlan& pl, const c3d_schedule
     f.ntiles = pix_tiles(items, (int)pl.n);
     HIP_TRY(launch_pix_tile_prefix(f.batch, f.nitems, s->tile_pre.p, st));
     f.tile_pre = s->tile_pre.p;
-    HIP_TRY(s->ks->filter(f, st));
+    HIP_TRY(use_quads(s, f, true)->filter(f, st));
     HIP_TRY(launch_threshold(f, s->need.p, s->plane2.p, npix, st));
     if (timed) MARK(-1);
     return C3D_OK;
@@ -1423,7 +1462,7 @@ int c3d_pm_densify_learned(c3d_pm_session* s, c3d_init_net* net, const uint32_t*
     f.ntiles = pix_tiles(items.data(), (int)items.size());
     HIP_TRY(launch_pix_tile_prefix(f.batch, f.nitems, s->tile_pre.p, st));
     f.tile_pre = s->tile_pre.p;
-    HIP_TRY(s->ks->filter(f, st));
+    HIP_TRY(use_quads(s, f, true)->filter(f, st));
     HIP_TRY(launch_threshold(f, s->need.p, s->plane2.p, npix, st));
     MARK(-1);
     HIP_TRY(hipEventSynchronize(s->marks[s->marks_used - 1]));
@@ -1653,22 +1692,25 @@ int c3d_pm_autotune(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32
     k.run_id = 0x7FFFFFFF;
     k.random_init = 1;
     k.ntiles = pix_tiles(items.data(), (int)items.size());
-    HIP_TRY(s->ks->eval(k, 1, st));
+    const KernelSet* ks = use_quads(s, k, run_quad8(s, k, items, 0));
+    HIP_TRY(ks->eval(k, 1, st));
     const int cand[C3D_TILE_SHAPES][2] = {{1, 1}, {2, 1}, {4, 1}, {4, 2}};
     double ms[C3D_TILE_SHAPES] = {};
     int bestc = 0;
     for (int c = 0; c < C3D_TILE_SHAPES; ++c) {
         KParams h = k;
         h.random_init = 0;
+        ks = use_quads(s, h, run_quad8(s, k, items, 0));
         h.ntiles = half_tiles(items.data(), (int)items.size(), cand[c][0], cand[c][1]);
         HIP_TRY(launch_half_tile_prefix(h.batch, h.nitems, cand[c][0], cand[c][1], s->tile_pre.p, st));
         h.tile_pre = s->tile_pre.p;
         for (int it = 0; it < 3; ++it) {
             iteration_constants(s->pm_copy, false, (uint32_t)it, h);
+            if (it == 1) ks = use_quads(s, h, run_quad8(s, k, items, 1));
             if (it == 1) HIP_TRY(hipEventRecord(s->ev[0], st));
             for (int color = 0; color < 2; ++color) {
                 h.color = color;
-                HIP_TRY(s->ks->half(h, cand[c][0], cand[c][1], st));
+                HIP_TRY(ks->half(h, cand[c][0], cand[c][1], st));
             }
         }
         HIP_TRY(hipEventRecord(s->ev[1], st));
@@ -1766,7 +1808,7 @@ int c3d_pm_pair_costs(c3d_pm_session* s, uint32_t level, uint32_t view, uint32_t
     HIP_TRY(hipMemcpyAsync(s->q_planes.p, planes, (size_t)nq * sizeof(float4), hipMemcpyHostToDevice, st));
     std::vector<BatchItem> none;
     KParams k = params_for(s, level, false, none, 1);
-    HIP_TRY(s->ks->pair_costs(k, (int)view, (int)slot, (int)nq, s->q_xy.p, s->q_planes.p, s->q_out.p, st));
+    HIP_TRY(use_quads(s, k, true)->pair_costs(k, (int)view, (int)slot, (int)nq, s->q_xy.p, s->q_planes.p, s->q_out.p, st));
     HIP_TRY(hipMemcpyAsync(costs, s->q_out.p, (size_t)nq * sizeof(float), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     return C3D_OK;
