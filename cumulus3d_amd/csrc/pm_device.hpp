@@ -251,6 +251,23 @@ __device__ __forceinline__ float c3d_expf(float x) {
     return x != x ? x : e;
 }
 
+// c3d_expf(-t) for t >= 0 (or NaN) in 15 instead of 25 operations: no upper bound to keep, the lower one
+// by the last select alone, and the power of two applied by exponent (p 2^n is normal, so exact).
+__device__ __forceinline__ float expf_down(float t) {
+    const float n = rintf(-t * 1.44269504088896341f);
+    float r = fmaf(-n, 0.693145751953125f, -t);
+    r = fmaf(-n, 1.42860677e-06f, r);
+    float p = 1.98412698e-04f;
+    p = fmaf(p, r, 1.38888889e-03f);
+    p = fmaf(p, r, 8.33333333e-03f);
+    p = fmaf(p, r, 4.16666667e-02f);
+    p = fmaf(p, r, 1.66666667e-01f);
+    p = fmaf(p, r, 0.5f);
+    p = fmaf(p, r, 1.0f);
+    p = fmaf(p, r, 1.0f);
+    return t >= 86.0f ? 0.0f : __builtin_amdgcn_ldexpf(p, (int)n);
+}
+
 // sin and cos: quadrant reduction, Taylor polynomials on |r| <= pi/4.
 __device__ __forceinline__ void c3d_sincosf(float x, float& so, float& co) {
     float k = rintf(x * 0.636619772367581343f);
@@ -344,6 +361,7 @@ struct Win {
     static constexpr int WN = (2 * WR) / WSTEP + 1;
     static constexpr int WN2 = WN * WN;
     static constexpr int LAST = -WR + (WN - 1) * WSTEP;  // last sample offset
+    static constexpr bool HELD = WN2 <= 49;              // registers hold the weights
 };
 
 // Weighted statistics of the reference patch (patchmatch.cu:199-223): bilateral weights w_k in
@@ -352,7 +370,7 @@ struct Win {
 template <int WR, int WSTEP>
 struct RefWin {
     float ic, mu, W, iW, var;
-    float w[Win<WR, WSTEP>::WN2];
+    float w[Win<WR, WSTEP>::HELD ? Win<WR, WSTEP>::WN2 : 1];
 };
 
 // Reference image accessors: 0 outside the image.
@@ -375,12 +393,51 @@ struct RefTile {
 __device__ __forceinline__ float bilateral_weight(const KParams& P, float ic, float v, int dx, int dy) {
     float d = ic - v;
     float sp = (float)(dx * dx + dy * dy) * P.inv2s;
-    return c3d_expf(-fmaf(d * d, P.inv2c255, sp));
+    return expf_down(fmaf(d * d, P.inv2c255, sp));
+}
+
+// ref_stats where the weights are not held: formed again where they are used, row by row, the same values.
+template <int WR, int WSTEP, class REF>
+__device__ __forceinline__ void ref_stats_rows(const KParams& P, const REF& ref, int x, int y, RefWin<WR, WSTEP>& rw) {
+    constexpr int WN = Win<WR, WSTEP>::WN;
+    rw.ic = ref.at(x, y);
+    float W = 0.0f, S = 0.0f;
+#pragma unroll 1
+    for (int a = 0; a < WN; ++a) {
+        const int dy = -WR + a * WSTEP;
+#pragma unroll
+        for (int b = 0; b < WN; ++b) {
+            const int dx = -WR + b * WSTEP;
+            const float v = ref.at(x + dx, y + dy), w = bilateral_weight(P, rw.ic, v, dx, dy);
+            W += w;
+            S = fmaf(w, v, S);
+        }
+    }
+    const float mu = S / W;
+    float V = 0.0f;
+#pragma unroll 1
+    for (int a = 0; a < WN; ++a) {
+        const int dy = -WR + a * WSTEP;
+#pragma unroll
+        for (int b = 0; b < WN; ++b) {
+            const int dx = -WR + b * WSTEP;
+            const float v = ref.at(x + dx, y + dy), dk = v - mu;
+            V = fmaf(bilateral_weight(P, rw.ic, v, dx, dy) * dk, dk, V);
+        }
+    }
+    rw.mu = mu;
+    rw.W = W;
+    rw.iW = 1.0f / W;
+    rw.var = V / W;
 }
 
 template <int WR, int WSTEP, class REF>
 __device__ __forceinline__ void ref_stats(const KParams& P, const REF& ref, int x, int y, RefWin<WR, WSTEP>& rw) {
     constexpr int WN = Win<WR, WSTEP>::WN;
+    if constexpr (!Win<WR, WSTEP>::HELD) {
+        ref_stats_rows<WR, WSTEP>(P, ref, x, y, rw);
+        return;
+    }
     rw.ic = ref.at(x, y);
     float W = 0.0f, S = 0.0f;
 #pragma unroll
@@ -393,7 +450,7 @@ __device__ __forceinline__ void ref_stats(const KParams& P, const REF& ref, int 
             float v = ref.at(x + dx, y + dy);
             float d = rw.ic - v;
             float sp = (float)(dx * dx + dy * dy) * P.inv2s;
-            float w = c3d_expf(-fmaf(d * d, P.inv2c255, sp));
+            float w = expf_down(fmaf(d * d, P.inv2c255, sp));
             rw.w[k] = w;
             W += w;
             S = fmaf(w, v, S);
@@ -617,19 +674,26 @@ __device__ __forceinline__ void window_sums(const RefWin<WR, WSTEP>& rw, const R
     }
 }
 
-// window_sums with CHECK as a loop over groups of CH samples that recomputes the bilateral weights;
-// same values and order. Windows that need the check are rare (0.4 to 2 % of a wave's windows have
+// window_sums as a loop over the rows, each in groups of CH samples whose gathers are issued together,
+// that forms the bilateral weights again; same values and order. Two uses:
+// Windows of more than 49 samples (the quality profile's (5, 1)), whose weights registers cannot
+// hold: with the window known at compile time the offsets are constants, the reference reads carry
+// theirs as immediates and the samples in front of the source need no check. 2 iterations of 3 views
+// with 3 sources against the kernels of any radius: 641 x 479 13.3 -> 12.1 ms, geometric 16.4 ->
+// 11.5 ms, 1281 x 959 46.8 -> 37.5 ms. Half of a sample's VALU instructions are its weight.
+// Whole rows at three waves per SIMD; two waves measured 12.8 ms, four (spills) 12.4 ms, half
+// rows at four 13.0 ms.
+// Windows with CHECK. Windows that need the check are rare (0.4 to 2 % of a wave's windows have
 // such a lane, over runs on 1920 x 1080 and 960 x 540 views). A second unrolled copy of the window
 // beside the first one costs registers all the same (the compiler hoists what the two have in
 // common above the branch: 247 VGPRs instead of 192 in the photometric half step) and drains the
 // first gathers there. Groups of one sample measured 2 % slower on one 960 x 540 view, of six
 // 3 % slower on 9 views of 1920 x 1080 (spills).
-template <int WR, int WSTEP, class REF>
-__device__ __forceinline__ void window_sums_behind(const KParams& P, const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y,
+template <int WR, int WSTEP, bool CHECK, int CH, class REF>
+__device__ __forceinline__ void window_rows(const KParams& P, const RefWin<WR, WSTEP>& rw, const REF& ref, int x, int y,
                                                    const QuadTable& qt, const float* H,
                                                    float& Ss, float& SSs, float& IS) {
     constexpr int WN = Win<WR, WSTEP>::WN;
-    constexpr int CH = 3;
     Ss = 0.f;
     SSs = 0.f;
     IS = 0.f;
@@ -653,7 +717,7 @@ __device__ __forceinline__ void window_sums_behind(const KParams& P, const RefWi
             for (int g = 0; g < CH; ++g) {
                 if (WN % CH != 0 && b0 + g >= WN) break;
                 const int dx = -WR + (b0 + g) * WSTEP;
-                const float sv = zs[g] > 1e-8f ? quad_lerp(qv[g], fx[g], fy[g]) : 0.0f;
+                const float sv = !CHECK || zs[g] > 1e-8f ? quad_lerp(qv[g], fx[g], fy[g]) : 0.0f;
                 const float iv = ref.at(x + dx, y + dy);
                 const float sp = sv - rw.ic;
                 const float ws = bilateral_weight(P, rw.ic, iv, dx, dy) * sp;
@@ -686,12 +750,15 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
     const bool all_front = fmaf(H[6], lo, za) > 1e-8f && fmaf(H[6], hi, za) > 1e-8f && fmaf(H[6], lo, zb) > 1e-8f &&
                            fmaf(H[6], hi, zb) > 1e-8f;
     float Ss, SSs, IS;
-    if (all_front) {
+    if constexpr (!Win<WR, WSTEP>::HELD) {
+        if (all_front) window_rows<WR, WSTEP, false, Win<WR, WSTEP>::WN>(P, rw, ref, x, y, qt, H, Ss, SSs, IS);
+        else window_rows<WR, WSTEP, true, 3>(P, rw, ref, x, y, qt, H, Ss, SSs, IS);
+    } else if (all_front) {
         window_sums<WR, WSTEP, false, PIPE, AHEAD>(rw, ref, x, y, qt, H, Ss, SSs, IS);
     } else if constexpr (COPY) {
         window_sums<WR, WSTEP, true, PIPE, AHEAD>(rw, ref, x, y, qt, H, Ss, SSs, IS);
     } else {
-        window_sums_behind<WR, WSTEP>(P, rw, ref, x, y, qt, H, Ss, SSs, IS);
+        window_rows<WR, WSTEP, true, 3>(P, rw, ref, x, y, qt, H, Ss, SSs, IS);
     }
     const float iW = rw.iW;
     float mus = Ss * iW;
@@ -706,7 +773,7 @@ __device__ __forceinline__ float ncc_cost(const KParams& P, const RefWin<WR, WST
 
 // ---------------------------------------------------------------- windows of any radius
 
-// Windows too large for register-resident weights (any radius up to 20, step 1 or 2; the kernels
+// Windows without a compiled-in build (any radius up to 20, step 1 or 2; the kernels
 // instantiated with WR = 0 read the radius from KParams::wr): the bilateral weight of a sample is
 // recomputed where it is used, as the reference does for windows above 36 samples
 // (patchmatch.cu:47,153-165). Every operation and its order match the register-resident path, so
@@ -759,7 +826,8 @@ __device__ void ref_stats_dyn(const KParams& P, const REF& ref, int x, int y, in
     rw.var = V / W;
 }
 
-template <int WSTEP, bool CHUNK, class REF>
+constexpr int DYN_GROUP = 6;
+template <int WSTEP, class REF>
 __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& ref, const LevelDesc& S, const float* H, int x,
                               int y) {
     float z = H[8];
@@ -779,15 +847,27 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
         const float rz = fmaf(H[7], oy, H[8]);
         const float ru = fmaf(H[1], oy, H[2]);
         const float rv = fmaf(H[4], oy, H[5]);
-        if constexpr (!CHUNK) {
-#pragma unroll 2
-            for (int b = 0; b < wn; ++b) {
-                const int dxi = -wr + b * WSTEP;
-                const float ox = (float)dxi;
-                const float zz = fmaf(H[6], ox, rz);
-                const float r = rcp_sample(zz);
-                float sv = quad_sample(qt, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r);
-                sv = zz > 1e-8f ? sv : 0.0f;
+        // G samples from b0 on: their gathers are issued before the first is used (the barrier keeps
+        // the compiler from waiting for each in turn). Groups of six at three waves per SIMD against the
+        // loop over single samples at two, 2 iterations of 3 views with 3 sources: 641 x 479 window
+        // (7, 2) 8.0 -> 7.65 ms, geometric 10.3 -> 8.5 ms; (5, 1) 13.3 -> 12.5 and 16.4 -> 13.0 ms;
+        // 1281 x 959 (5, 1) 46.8 -> 41.5 ms. Groups of four: 13.1, 13.5 and 43.4 ms for the last three.
+        auto group = [&](int b0, auto g) {
+            constexpr int G = decltype(g)::value;
+            QuadEntry qs[G];
+            float fx[G], fy[G], zs[G];
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const float ox = (float)(-wr + (b0 + i) * WSTEP);
+                zs[i] = fmaf(H[6], ox, rz);
+                const float r = rcp_sample(zs[i]);
+                qs[i] = quad_fetch(qt, fmaf(H[0], ox, ru) * r, fmaf(H[3], ox, rv) * r, fx[i], fy[i]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int dxi = -wr + (b0 + i) * WSTEP;
+                const float sv = zs[i] > 1e-8f ? quad_lerp(qs[i], fx[i], fy[i]) : 0.0f;
                 const float iv = ref.at(x + dxi, y + dyi);
                 const float sp = sv - rw.ic;
                 const float ws = bilateral_weight(P, rw.ic, iv, dxi, dyi) * sp;
@@ -795,41 +875,16 @@ __device__ float ncc_cost_dyn(const KParams& P, const RefWinDyn& rw, const REF& 
                 SSs = fmaf(ws, sp, SSs);
                 IS = fmaf(ws, iv, IS);
             }
-            continue;
-        }
-        // chunks of four samples: the four gathers are issued before the first is consumed (the
-        // samples past the row's end in the last chunk repeat its last sample and are not summed);
-        // faster in the geometric builds, slower in the photometric one
-        for (int b0 = 0; b0 < wn; b0 += 4) {
-            QuadEntry qs[4];
-            float fxs[4], fys[4], zs[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int b = b0 + u < wn ? b0 + u : wn - 1;
-                const float ox = (float)(-wr + b * WSTEP);
-                const float zz = fmaf(H[6], ox, rz);
-                const float r = rcp_sample(zz);
-                const float su = fmaf(H[0], ox, ru) * r, sw = fmaf(H[3], ox, rv) * r;
-                zs[u] = zz;
-                qs[u] = quad_fetch(qt, su, sw, fxs[u], fys[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int b = b0 + u;
-                if (b >= wn) break;
-                const int dxi = -wr + b * WSTEP;
-                const QuadEntry q = qs[u];
-                const float ax = fxs[u], ay = fys[u];
-                float sv = quad_lerp(q, ax, ay);
-                sv = zs[u] > 1e-8f ? sv : 0.0f;
-                const float iv = ref.at(x + dxi, y + dyi);
-                const float sp = sv - rw.ic;
-                const float ws = bilateral_weight(P, rw.ic, iv, dxi, dyi) * sp;
-                Ss += ws;
-                SSs = fmaf(ws, sp, SSs);
-                IS = fmaf(ws, iv, IS);
-            }
-        }
+        };
+        int b = 0;
+#pragma unroll 1
+        for (; b + DYN_GROUP <= wn; b += DYN_GROUP) group(b, std::integral_constant<int, DYN_GROUP>{});
+        const int rest = wn - b;
+        if (rest == 1) group(b, std::integral_constant<int, 1>{});
+        else if (rest == 2) group(b, std::integral_constant<int, 2>{});
+        else if (rest == 3) group(b, std::integral_constant<int, 3>{});
+        else if (rest == 4) group(b, std::integral_constant<int, 4>{});
+        else if (rest == 5) group(b, std::integral_constant<int, 5>{});
     }
     const float iW = rw.iW;
     float mus = Ss * iW;
@@ -849,11 +904,11 @@ __device__ __forceinline__ void ref_stats_any(const KParams& P, const REF& ref, 
     else ref_stats_dyn<WSTEP>(P, ref, x, y, wr, rw);
 }
 
-template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool CHUNK = false, bool AHEAD = false, bool COPY = false, class REF>
+template <int WR, int WSTEP, int PIPE = WINDOW_PIPE, bool AHEAD = false, bool COPY = false, class REF>
 __device__ __forceinline__ float ncc_cost_any(const KParams& P, const RefWinT<WR, WSTEP>& rw, const REF& ref, const LevelDesc& S,
                                               const float* H, int x, int y) {
     if constexpr (WR > 0) return ncc_cost<WR, WSTEP, PIPE, AHEAD, COPY>(P, rw, ref, S, H, x, y);
-    else return ncc_cost_dyn<WSTEP, CHUNK>(P, rw, ref, S, H, x, y);
+    else return ncc_cost_dyn<WSTEP>(P, rw, ref, S, H, x, y);
 }
 
 // Forward-backward reprojection error through the source depth snapshot (patchmatch.cu:292-314).

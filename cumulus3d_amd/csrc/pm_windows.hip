@@ -76,7 +76,7 @@ __device__ __forceinline__ float pair_cost_h(const KParams& P, const RefWinT<WR,
     // geometric runs: the snapshot depth is fetched before the NCC window and used after it
     GeoFetch gf{0.f, 0.f, 0.f, false};
     if constexpr (GEO) gf = geo_fetch(P, R, S, pr, x, y, h.w);
-    if (homography(R, lp, ifx, ify, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP, PIPE, GEO, AHEAD, COPY>(P, rw, ref, S, H, x, y);
+    if (homography(R, lp, ifx, ify, (float)x, (float)y, h.w, xyz(h), H)) c = ncc_cost_any<WR, WSTEP, PIPE, AHEAD, COPY>(P, rw, ref, S, H, x, y);
     geo = GEO ? fminf(geo_finish(R, S, pr, x, y, gf), P.gmax) : 0.f;
     return c;
 }
@@ -99,6 +99,7 @@ __device__ __forceinline__ float pair_cost_h(const KParams& P, const RefWinT<WR,
 constexpr int FEW_WAVES = 16384;
 template <int WR, int WSTEP>
 constexpr int half_waves(bool few) {
+    if (WR == 0 || !Win<(WR > 0 ? WR : 1), WSTEP>::HELD) return 3;  // rows or groups of samples (window_rows, ncc_cost_dyn)
     return (!few && WR > 0 && Win<(WR > 0 ? WR : 1), WSTEP>::WN2 <= 36) ? 3 : 2;
 }
 
@@ -648,10 +649,11 @@ static constexpr KernelSet make_set() {
 
 // Window variants compiled into the library (radius, step): the fast profile (5, 2) and the
 // variants of the reference's window report (patchmatch_gpu.rs:164) whose window holds at most
-// 49 samples, with the bilateral weights in registers; every other radius up to 20 (the quality
-// profile's (5, 1) among them) runs the any-radius kernels (wr = 0 below) of its step.
+// 49 samples, with the bilateral weights in registers; the quality profile's (5, 1), which forms them
+// row by row (window_rows); every other radius up to 20 runs the any-radius kernels (wr = 0 below)
+// of its step.
 static const KernelSet kSets[] = {make_set<5, 2>(), make_set<4, 2>(), make_set<3, 2>(), make_set<2, 2>(), make_set<3, 1>(),
-                                  make_set<2, 1>(), make_set<1, 1>()};
+                                  make_set<2, 1>(), make_set<1, 1>(), make_set<5, 1>()};
 static const KernelSet kAny[] = {make_set<0, 1>(), make_set<0, 2>()};
 
 const KernelSet* kernel_set(int wr, int wstep, bool any_radius) {
