@@ -597,8 +597,8 @@ def plain_main(args):
     half_ms = sum(t.half_kernel_ms for t in tms) / sum(t.half_launches for t in tms)
     default_zone7 = (not batched and nviews == 7 and (args.width, args.height) == (1920, 1080) and args.photometric_iters == 7
                      and args.geometric_rounds == 1 and args.geometric_iters == 2 and tuple(args.window) == (5, 2))
-    # the windows built with register-held weights; every other one runs the any-radius build
-    reg_windows = {(5, 2), (4, 2), (3, 2), (2, 2), (3, 1), (2, 1), (1, 1)}
+    # the windows compiled in; every other one runs the any-radius build
+    reg_windows = {(5, 2), (4, 2), (3, 2), (2, 2), (3, 1), (2, 1), (1, 1), (5, 1)}
     kernel_name = (f"k_half<{inp.pm.window_radius},{inp.pm.window_step}>"
                    if (inp.pm.window_radius, inp.pm.window_step) in reg_windows else f"k_half<any radius,{inp.pm.window_step}>")
     roof, roof_valu = roofline_objects(kernel_name, avg_bytes, flop, half_ms, K_HALF_TRAFFIC.get(("zone7", tuple(shape))) if default_zone7 else None)

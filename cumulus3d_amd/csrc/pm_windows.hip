@@ -88,15 +88,17 @@ __device__ __forceinline__ float pair_cost_h(const KParams& P, const RefWinT<WR,
 // refinement candidates of index j modulo TPP, and the costs are exchanged; every decision is then
 // taken on all of them from the same values in the same order, so the results are those of one
 // lane per pixel.
-// FEW: the build for launches of up to FEW_WAVES waves, at two waves per SIMD, with more gathers in
+// FEW: the build for launches of up to few_waves() waves, at two waves per SIMD, with more gathers in
 // flight and the unrolled copy of the window (see ncc_cost). Its waves are a quarter shorter by
 // themselves, and a launch of a few rounds ends with its last waves: one view of 960 x 540 (4,080
 // waves) takes 2.35 instead of 2.51 ms for 2 iterations with 3 sources, 1920 x 1080 (16,200) 7.33
 // instead of 7.52. Two such views (32,400) tie, and from there the three waves per SIMD of the
 // other build win: 9 views of 1920 x 1080 with 6 sources 22.2 -> 20.0 ms a half step. What binds it
 // is the issue of VALU instructions, which three waves keep busier (3.8 instead of 4.2 cycles an
-// instruction; 2.4 of 3 wave slots taken on average).
-constexpr int FEW_WAVES = 16384;
+// instruction; 2.4 of 3 wave slots taken on average). Geometric launches cross over earlier: 12 views
+// of 480 x 270 (12,648 waves) with 4 sources take 11.4 ms for 3 iterations in the FEW build and 10.9
+// in the other, 1280 x 720 (7,200) 6.2 ms in either, where the photometric ones take 4.8 and 5.1.
+constexpr int few_waves(bool geo) { return geo ? 8192 : 16384; }
 template <int WR, int WSTEP>
 constexpr int half_waves(bool few) {
     if (WR == 0 || !Win<(WR > 0 ? WR : 1), WSTEP>::HELD) return 3;  // rows or groups of samples (window_rows, ncc_cost_dyn)
@@ -603,8 +605,9 @@ static hipError_t launch_half(const KParams& P0, int rows, int tpp, hipStream_t 
     P.wv_stride = rows * 64;
     size_t lds = (size_t)P.wv_stride * (P.max_nsrc > 0 ? P.max_nsrc : 1) * sizeof(float);
     if (WR == 0) lds += half_tile_bytes(P.wr, rows, tpp);
-    const bool few = P.ntiles * rows <= FEW_WAVES;
-    if (rows == 1 && tpp == 1 && few) launch_half_rows<WR, WSTEP, 1, 1, true>(P, lds, s);
+    constexpr bool HELD = WR > 0 && Win<(WR > 0 ? WR : 1), WSTEP>::HELD;  // else both builds are one
+    const bool few = HELD && P.ntiles * rows <= few_waves(P.geometric);
+    if (rows == 1 && tpp == 1 && few) launch_half_rows<WR, WSTEP, 1, 1, HELD>(P, lds, s);
     else if (rows == 1 && tpp == 1) launch_half_rows<WR, WSTEP, 1, 1, false>(P, lds, s);
     else if (rows == 1 && tpp == 2) launch_half_rows<WR, WSTEP, 1, 2, true>(P, lds, s);
     else if (rows == 1 && tpp == 4) launch_half_rows<WR, WSTEP, 1, 4, true>(P, lds, s);

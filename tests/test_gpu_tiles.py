@@ -43,3 +43,28 @@ def test_block_edges_bit_exact(sizes):
                 assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32)), (rows, tpp)
         for a, b in zip(gc, rc):
             assert np.array_equal(a, b), (rows, tpp)
+
+
+@pytest.mark.parametrize("width", [1008, 1024, 1040])  # two views: 8064, 8192 and 8320 waves
+def test_builds_agree_across_the_geometric_wave_count(width):
+    """One-row workgroups take the two-wave build of the half step up to 8192 waves of a geometric run and
+    the three-wave build above; two-row workgroups always take the latter. Same states."""
+    sizes = [(width, 512)] * 2
+    sc = scenes.make_mixed_scene(scenes.oblique_rig(2), sizes, seed=29)
+    pmp, fl = abi.fast_profile()
+    inp = scenes.kernel_input(sc, [[1], [0]], [(15.0, 120.0)] * 2, pmp, fl)
+    outs = []
+    for rows in (1, 2):
+        opts = abi.c3d_pm_options()
+        opts.tile_rows, opts.threads_per_pixel = rows, 1
+        be = pm.HipPatchMatch(0, opts)
+        with be.begin(inp) as s:
+            st = [abi.ViewState(w, h) for w, h in sizes]
+            s.run([0, 1], st, abi.run_params(0, False, True, 1, 1, False))
+            snap = abi.DepthSnapshot(5, 0, [x.depth.copy() for x in st])
+            s.run([0, 1], st, abi.run_params(0, True, False, 1, 2, False), snap)
+            outs.append(st)
+        be.close()
+    for a, b in zip(*outs):
+        for x, y in ((a.depth, b.depth), (a.normal, b.normal), (a.cost, b.cost)):
+            assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
