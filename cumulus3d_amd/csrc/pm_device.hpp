@@ -108,22 +108,36 @@ struct KParams {
 // in that L2, and the runs are dealt to the XCDs in turn, so that every XCD gets its share of the
 // costly and of the cheap parts of each view. (One contiguous eighth of the tiles per XCD left
 // XCDs idle while the one with the costliest eighth finished: 1.7 of 2 wave slots per SIMD were
-// taken on average. 9 views of 1920 x 1080 with 6 sources: half step 24.9 -> 23.5 ms; 2 such
-// views from a random start: 38.8 -> 35.3 ms a run of 3 iterations. Runs of 4 and 8 tiles measured
-// 3 and 2 % slower in the half step, 64 and 256 1 % slower.) The tiles after the last whole round
-// keep their order.
-constexpr int XCD_RUN = 16;
+// taken on average.) In the half step a run is a square of 8 x 8 blocks (HALF_BAND), 128 x 64 pixels.
+// Each round of 8 runs starts at another XCD, scattered by a multiplicative hash: without it a width
+// of a whole or half number of rounds gives each XCD the same columns of every view. Measured against
+// runs of 16 tiles of one row: half step of 9 views of 1920 x 1080 with 6 sources 17.91 -> 17.72 ms; 2
+// such views from a random start, 3 iterations 31.1 -> 30.15 ms; 9 views of up to 1283 x 717,
+// geometric, 24.5 -> 24.05 ms; 12 views of 960 x 540 over 3 scales 218.6 -> 217.0 ms (234 ms without
+// the scattering). Runs of 32 tiles, 4 x 8 or 8 x 4, gained less (17.92 and 17.86 ms; 30.9 and 31.2 ms).
+// The tiles after the last whole round keep their order.
+constexpr int XCD_RUN = 64;
+constexpr int HALF_BAND = 8;
 __device__ __forceinline__ int xcd_tile(int bid, int n) {
     const int nx = 8;
     if (bid >= n - n % (nx * XCD_RUN)) return bid;
-    const int x = bid % nx, k = bid / nx;
-    return (k / XCD_RUN * nx + x) * XCD_RUN + k % XCD_RUN;
+    const int k = bid / nx, round = k / XCD_RUN;
+    const int x = (bid + (int)((uint32_t)round * 0x9E3779B1u >> 29)) % nx;
+    return (round * nx + x) * XCD_RUN + k % XCD_RUN;
+}
+
+// Tile tl of an item of tx x ty tiles: row by row, or (band > 1) column by column in bands of that many
+// rows.
+__device__ __forceinline__ void tile_origin(int tl, int tx, int ty, int tw, int th, int band, int& x0, int& y0) {
+    const int b = tl / (band * tx), r = tl - b * band * tx, rows = min(band, ty - b * band);
+    x0 = r / rows * tw;
+    y0 = (b * band + r % rows) * th;
 }
 
 // Finds the batch item of flattened tile `t` for tiles of tw x th pixels; returns the item and
 // the tile's pixel origin, or false when t is past the last item.
 __device__ __forceinline__ bool locate_tile(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0,
-                                            int* item = nullptr) {
+                                            int band = 1, int* item = nullptr) {
     for (int i = 0; i < P.nitems; ++i) {
         BatchItem b = P.batch[i];
         int tx = (b.w + tw - 1) / tw, ty = (b.h + th - 1) / th;
@@ -131,8 +145,7 @@ __device__ __forceinline__ bool locate_tile(const KParams& P, int t, int tw, int
         if (t < n) {
             it = b;
             if (item) *item = i;
-            y0 = (t / tx) * th;
-            x0 = (t % tx) * tw;
+            tile_origin(t, tx, ty, tw, th, band, x0, y0);
             return true;
         }
         t -= n;
@@ -143,7 +156,7 @@ __device__ __forceinline__ bool locate_tile(const KParams& P, int t, int tw, int
 // locate_tile through the launch's tile offsets (P.tile_pre, built for the same tw x th): a binary
 // search over the items instead of a linear one. The last item whose first tile is at or before t
 // holds it (items without tiles share their successor's offset and are passed over).
-__device__ __forceinline__ bool locate_tile_pre(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0) {
+__device__ __forceinline__ bool locate_tile_pre(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0, int band) {
     const int* pre = P.tile_pre;
     if (t >= pre[P.nitems]) return false;
     int lo = 0, hi = P.nitems - 1;
@@ -155,15 +168,14 @@ __device__ __forceinline__ bool locate_tile_pre(const KParams& P, int t, int tw,
     it = P.batch[lo];
     const int tl = t - pre[lo];
     const int tx = (it.w + tw - 1) / tw;
-    y0 = (tl / tx) * th;
-    x0 = (tl % tx) * tw;
+    tile_origin(tl, tx, (it.h + th - 1) / th, tw, th, band, x0, y0);
     return true;
 }
 
 // The tile's item and pixel origin through P.tile_pre when the launch provides it (built for the
 // same tw x th), else by the linear search.
-__device__ __forceinline__ bool find_tile(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0) {
-    return P.tile_pre ? locate_tile_pre(P, t, tw, th, it, x0, y0) : locate_tile(P, t, tw, th, it, x0, y0);
+__device__ __forceinline__ bool find_tile(const KParams& P, int t, int tw, int th, BatchItem& it, int& x0, int& y0, int band = 1) {
+    return P.tile_pre ? locate_tile_pre(P, t, tw, th, it, x0, y0, band) : locate_tile(P, t, tw, th, it, x0, y0, band);
 }
 
 // ---------------------------------------------------------------- tile shapes

@@ -393,9 +393,9 @@ void iteration_constants(const c3d_pm_params& pm, bool geometric, uint32_t t, KP
 
 // Which of the two quad tables a run takes. The 8-byte entries save 4 of a sample's 33 instructions and
 // double what the samples touch. Where neighbouring pixels sample near each other that pays: half
-// step of 9 views of 1920 x 1080 with 6 sources from the network's planes 19.3 -> 17.9 ms, 24
-// geometric views of 480 x 270 25.7 -> 24.7 ms a run, evaluation and read-out filter of the 9 views
-// 3.07 -> 2.75 ms. A run from random planes samples all over its sources, waits for L2 misses, and
+// step of 9 views of 1920 x 1080 with 6 sources from the network's planes 19.3 -> 17.9 ms, a
+// geometric run over 9 views of up to 1283 x 717 with 5 sources 25.7 -> 24.7 ms, read-out filter of the
+// 9 large views 3.07 -> 2.75 ms. A run from random planes samples all over its sources, waits for L2 misses, and
 // loses unless the tables are small, first iteration and later ones (6 views, 6 sources, 4-byte and
 // 8-byte): 1920 x 1080 43.1 and 54.1, 24.6 and 25.3 ms; 960 x 540 9.9 and 12.0, 6.41 and 6.15 ms;
 // 480 x 270 (12 views) 5.9 and 5.9, 4.1 and 3.7 ms.

@@ -130,7 +130,7 @@ void k_half(KParams P) {
 
     BatchItem it;
     int px0, py0;
-    if (!find_tile(P, xcd_tile(blockIdx.x, P.ntiles), BW, BH, it, px0, py0)) return;
+    if (!find_tile(P, xcd_tile(blockIdx.x, P.ntiles), BW, BH, it, px0, py0, HALF_BAND / ROWS)) return;
     const LevelDesc R = P.lv[it.view * P.nlevels + P.level];
     const int w = it.w, h = it.h;
     {

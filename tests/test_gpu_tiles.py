@@ -68,3 +68,31 @@ def test_builds_agree_across_the_geometric_wave_count(width):
     for a, b in zip(*outs):
         for x, y in ((a.depth, b.depth), (a.normal, b.normal), (a.cost, b.cost)):
             assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
+
+
+@pytest.mark.parametrize("sizes", [
+    [(512, 128), (496, 128), (528, 136)],  # 512 tiles (a whole round of runs of 64), fewer, more
+    [(130, 200), (17, 300), (300, 17)],    # bands of 8 rows of blocks with a rest, one column, under one band
+])
+def test_bands_of_blocks_bit_exact(sizes):
+    import oracle
+
+    sc = scenes.make_mixed_scene(scenes.oblique_rig(3), sizes, seed=37)
+    pmp, fl = abi.fast_profile()
+    inp = scenes.kernel_input(sc, [[1, 2], [0, 2], [0, 1]], [(15.0, 120.0)] * 3, pmp, fl)
+
+    def run(engine):
+        st = [abi.ViewState(w, h) for w, h in sizes]
+        engine.run([0, 1, 2], st, abi.run_params(0, False, True, 2, 1, False))
+        return [x for s in st for x in (s.depth, s.normal, s.cost)]
+
+    ref = run(oracle.Oracle(inp, threads=16))
+    for rows, tpp in [(0, 0)] + list(abi.TILE_SHAPES):
+        opts = abi.c3d_pm_options()
+        opts.tile_rows, opts.threads_per_pixel = rows, tpp
+        be = pm.HipPatchMatch(0, opts)
+        with be.begin(inp) as s:
+            got = run(s)
+        be.close()
+        for a, b in zip(got, ref):
+            assert np.array_equal(np.asarray(a).view(np.uint32), np.asarray(b).view(np.uint32)), (rows, tpp)
