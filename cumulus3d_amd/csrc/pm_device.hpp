@@ -115,15 +115,19 @@ struct KParams {
 // such views from a random start, 3 iterations 31.1 -> 30.15 ms; 9 views of up to 1283 x 717,
 // geometric, 24.5 -> 24.05 ms; 12 views of 960 x 540 over 3 scales 218.6 -> 217.0 ms (234 ms without
 // the scattering). Runs of 32 tiles, 4 x 8 or 8 x 4, gained less (17.92 and 17.86 ms; 30.9 and 31.2 ms).
+// Windows whose weights are formed again wait less for L2 and more for the last XCD: they keep runs of
+// 16 of one row (3 views of 641 x 479, window (5, 1): 12.25 against 12.6 ms).
 // The tiles after the last whole round keep their order.
 constexpr int XCD_RUN = 64;
+constexpr int XCD_RUN_ROW = 16;
 constexpr int HALF_BAND = 8;
+template <int RUN = XCD_RUN>
 __device__ __forceinline__ int xcd_tile(int bid, int n) {
     const int nx = 8;
-    if (bid >= n - n % (nx * XCD_RUN)) return bid;
-    const int k = bid / nx, round = k / XCD_RUN;
+    if (bid >= n - n % (nx * RUN)) return bid;
+    const int k = bid / nx, round = k / RUN;
     const int x = (bid + (int)((uint32_t)round * 0x9E3779B1u >> 29)) % nx;
-    return (round * nx + x) * XCD_RUN + k % XCD_RUN;
+    return (round * nx + x) * RUN + k % RUN;
 }
 
 // Tile tl of an item of tx x ty tiles: row by row, or (band > 1) column by column in bands of that many

@@ -130,7 +130,8 @@ void k_half(KParams P) {
 
     BatchItem it;
     int px0, py0;
-    if (!find_tile(P, xcd_tile(blockIdx.x, P.ntiles), BW, BH, it, px0, py0, HALF_BAND / ROWS)) return;
+    constexpr bool HELD = WR > 0 && Win<(WR > 0 ? WR : 1), WSTEP>::HELD;
+    if (!find_tile(P, xcd_tile<HELD ? XCD_RUN : XCD_RUN_ROW>(blockIdx.x, P.ntiles), BW, BH, it, px0, py0, HELD ? HALF_BAND / ROWS : 1)) return;
     const LevelDesc R = P.lv[it.view * P.nlevels + P.level];
     const int w = it.w, h = it.h;
     {
