@@ -1,5 +1,5 @@
 """Sizes at the edges of the half step's pixel blocks (16 x 8 pixels a wave with one lane per pixel)
-and of the runs of 16 tiles that are dealt to the 8 XCDs (128 tiles a round): the engine equals the
+and of the runs of 16 or 64 tiles that are dealt to the 8 XCDs (128 or 512 tiles a round): the engine equals the
 oracle bit for bit under every workgroup shape."""
 import numpy as np
 import pytest
