@@ -356,16 +356,16 @@ void k_half(KParams P) {
     // skipped. The accepted planes and costs are unchanged.
     // With several lanes per pixel each lane costs its candidates against the step-2 best (a
     // candidate that reaches it cannot be accepted later either, the best only decreasing), then
-    // all of them accept in candidate order from the exchanged costs.
+    // all of them accept in candidate order from the exchanged costs: a skipped candidate's is its
+    // partial sum, at or above the step-2 best (which has no upper bound: it grows with lambda gmax).
     const bool early = P.lambda >= 0.f && (!GEO || P.gmax >= 0.f);
     float ccs[7];
 #pragma unroll
-    for (int q = 0; q < 7; ++q) ccs[q] = 3.f;  // above any cost: not accepted
+    for (int q = 0; q < 7; ++q) ccs[q] = 0.f;  // each is set by the lane that costs it
 #pragma nounroll
     for (int c = sub; c < ncand; c += TPP) {
         const float4 hc = cand[c * NT];
         float cc = 2.f;
-        bool out = false;
         if (den > 0.f) {
             float nm = 0.f;
 #pragma nounroll
@@ -377,10 +377,7 @@ void k_half(KParams P) {
                 float g;
                 float m = pair_cost_h<WR, WSTEP, GEO, PIPE, AHEAD, FEW>(P, rw, ref, R, S, pr, lps[j], ifx, ify, x, y, hc, g);
                 nm += wj * (m + P.lambda * g);
-                if (early && nm / den >= bcost) {
-                    out = true;
-                    break;
-                }
+                if (early && nm / den >= bcost) break;
             }
             cc = nm / den;
         }
@@ -392,7 +389,7 @@ void k_half(KParams P) {
         } else {
 #pragma unroll
             for (int q = 0; q < 7; ++q)
-                if (q == c) ccs[q] = out ? 3.f : cc;
+                if (q == c) ccs[q] = cc;
         }
     }
     if constexpr (TPP > 1) {
