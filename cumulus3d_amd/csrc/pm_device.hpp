@@ -42,7 +42,7 @@ struct LevelDesc {
     long long goff;  // byte offset of the u8 image
     float fx, fy, cx, cy;
     float ifx, ify;   // 1 / fx, 1 / fy
-    int plain, pad1;  // both focal lengths lie where division by them may go through div_exact
+    int plain, pad1;  // k lies where a pixel's (u - c) / f may go through div_exact
 };
 
 struct PairRec {
@@ -331,7 +331,8 @@ __device__ __forceinline__ float rcp_sample(float z) {
 // the same bits as IEEE division and sqrtf in 3, 3 and 5 instructions; the compiler's sequences,
 // which also serve the ends of the exponent range, take 10, 10 and 13. inv_exact and sqrt_exact equal
 // the IEEE results on every mantissa of one and of two binades (measured on the device). For
-// arguments and results between 2^-100 and 2^100; callers keep IEEE division for the rest.
+// arguments and results between 2^-100 and 2^100 (and a = 0); callers keep IEEE division for the rest.
+// An infinite numerator or quotient gives NaN, not infinity.
 __device__ __forceinline__ float inv_exact(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
     return fmaf(r, fmaf(-x, r, 1.0f), r);
@@ -948,7 +949,7 @@ __device__ __forceinline__ GeoFetch geo_fetch(const KParams& P, const LevelDesc&
     float zj = pr.r[6] * X.x + pr.r[7] * X.y + pr.r[8] * X.z + pr.t[2];
     if (!(zj > 1e-8f)) return g;
     float u, v;
-    if (zj < EXACT_HI) {
+    if (zj < EXACT_HI) {  // an overflow is outside the source as NaN too
         const float iz = inv_exact(zj);
         u = div_exact(S.fx * xj, zj, iz) + S.cx;
         v = div_exact(S.fy * yj, zj, iz) + S.cy;
@@ -977,14 +978,16 @@ __device__ __forceinline__ float geo_finish(const LevelDesc& R, const LevelDesc&
     float Yy = pr.r[1] * q.x + pr.r[4] * q.y + pr.r[7] * q.z;
     float Yz = pr.r[2] * q.x + pr.r[5] * q.y + pr.r[8] * q.z;
     if (!(Yz > 1e-8f)) return INF_ERR;
+    const float nx = R.fx * Yx, ny = R.fy * Yy;
     float ex, ey;
-    if (Yz < EXACT_HI) {
+    // numerators below 2^100 over a divisor above 1e-8: quotients below 2^127
+    if (fmaxf(Yz, fmaxf(fabsf(nx), fabsf(ny))) < EXACT_HI) {
         const float iz = inv_exact(Yz);
-        ex = div_exact(R.fx * Yx, Yz, iz) + R.cx - (float)x;
-        ey = div_exact(R.fy * Yy, Yz, iz) + R.cy - (float)y;
+        ex = div_exact(nx, Yz, iz) + R.cx - (float)x;
+        ey = div_exact(ny, Yz, iz) + R.cy - (float)y;
     } else {
-        ex = R.fx * Yx / Yz + R.cx - (float)x;
-        ey = R.fy * Yy / Yz + R.cy - (float)y;
+        ex = nx / Yz + R.cx - (float)x;
+        ey = ny / Yz + R.cy - (float)y;
     }
     return sqrtf(ex * ex + ey * ey);
 }

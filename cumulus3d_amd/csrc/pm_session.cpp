@@ -640,7 +640,8 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
             L.cy = li.k[3];
             L.ifx = 1.0f / L.fx;
             L.ify = 1.0f / L.fy;
-            L.plain = std::fabs(L.fx) > 0x1p-20f && std::fabs(L.fx) < 0x1p40f && std::fabs(L.fy) > 0x1p-20f && std::fabs(L.fy) < 0x1p40f;
+            auto plain = [](float f, float c) { return std::fabs(f) > 0x1p-20f && std::fabs(f) < 0x1p40f && std::fabs(c) < 0x1p40f; };
+            L.plain = plain(L.fx, L.cx) && plain(L.fy, L.cy);
         }
     auto bail = [&](int code) {
         c3d_pm_end(s);
