@@ -252,6 +252,14 @@ int check_views(c3d_pm_session* s, uint32_t level, const uint32_t* views, uint32
     return C3D_OK;
 }
 
+// One output array per view.
+template <class T>
+int check_outputs(T* const* out, uint32_t n) {
+    for (uint32_t i = 0; i < n; ++i)
+        if (!out[i]) return fail(C3D_INVALID_ARGUMENT, "null output array of view " + std::to_string(i));
+    return C3D_OK;
+}
+
 // Bundles views by the pixel and view budgets (patchmatch.rs:606-625): [start, end) pairs.
 std::vector<std::pair<uint32_t, uint32_t>> batches(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32_t level) {
     std::vector<std::pair<uint32_t, uint32_t>> out;
@@ -830,6 +838,8 @@ int c3d_pm_evaluate(c3d_pm_session* s, uint32_t level, const uint32_t* views, ui
     if (rc) return rc;
     rc = check_views(s, level, views, n, states);
     if (rc) return rc;
+    rc = check_outputs(costs, n);
+    if (rc) return rc;
     if (geometric) {
         rc = ensure_snapshot(s, snap, level);
         if (rc) return rc;
@@ -860,6 +870,8 @@ int c3d_pm_filter(c3d_pm_session* s, const uint32_t* views, uint32_t n, const c3
                   uint8_t* const* counts) {
     if (!s || !snap || (n && (!views || !states || !counts))) return fail(C3D_INVALID_ARGUMENT, "null argument");
     int rc = set_device(s->be);
+    if (rc) return rc;
+    rc = check_outputs(counts, n);
     if (rc) return rc;
     rc = ensure_snapshot(s, snap, snap->level);
     if (rc) return rc;
