@@ -219,10 +219,12 @@ struct c3d_pm_session {
     std::vector<long long> h_snap_lv;
     std::vector<uint8_t> h_need;
     // half-step workgroup shape: rows of pixel blocks and lanes per pixel (options.tile_rows and
-    // options.threads_per_pixel, or c3d_pm_autotune)
+    // options.threads_per_pixel, or c3d_pm_autotune). Launches that half_lanes gives more lanes than
+    // half_below take one-row workgroups with those instead: all with 0 (no shape given or tuned),
+    // none with 8 (given), those smaller than the launch that was timed (tuned).
     int half_rows = 1;
     int half_tpp = 1;
-    bool half_auto = true;  // neither was given or tuned: every run picks its lanes per pixel (half_lanes)
+    int half_below = 0;
     // the captured schedule (options.use_graph) and the key it was captured for
     hipGraphExec_t gexec = nullptr;
     std::vector<uint8_t> gkey;
@@ -443,10 +445,12 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
         e.tile_pre = s->tile_pre.p;
         HIP_TRY(ks->eval_color(e, st));
     }
-    const int tpp = s->half_auto ? half_lanes(items.data(), (int)items.size()) : s->half_tpp;
-    k.ntiles = half_tiles(items.data(), (int)items.size(), s->half_rows, tpp);
+    const int lanes = half_lanes(items.data(), (int)items.size());
+    const bool own = lanes <= s->half_below;
+    const int rows = own ? s->half_rows : 1, tpp = own ? s->half_tpp : lanes;
+    k.ntiles = half_tiles(items.data(), (int)items.size(), rows, tpp);
     if (iterations > 0) {
-        HIP_TRY(launch_half_tile_prefix(k.batch, k.nitems, s->half_rows, tpp, s->tile_pre.p, st));
+        HIP_TRY(launch_half_tile_prefix(k.batch, k.nitems, rows, tpp, s->tile_pre.p, st));
         k.tile_pre = s->tile_pre.p;
     }
     for (uint32_t t = 0; t < iterations; ++t) {
@@ -462,7 +466,7 @@ int launch_run(c3d_pm_session* s, KParams k, const std::vector<BatchItem>& items
                 }
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used], st));
             }
-            HIP_TRY(ks->half(k, s->half_rows, tpp, st));
+            HIP_TRY(ks->half(k, rows, tpp, st));
             if (timed) {
                 HIP_TRY(hipEventRecord(s->pool[s->pool_used + 1], st));
                 s->pool_used += 2;
@@ -741,7 +745,7 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     s->filter_copy = fl;
     s->half_tpp = be->opts.threads_per_pixel == 2 ? 2 : 1;
     s->half_rows = default_rows(be->opts.tile_rows, s->half_tpp);
-    s->half_auto = be->opts.tile_rows == 0 && be->opts.threads_per_pixel == 0;
+    s->half_below = be->opts.tile_rows == 0 && be->opts.threads_per_pixel == 0 ? 0 : 8;
     *out = s;
     return C3D_OK;
 }
@@ -1707,15 +1711,18 @@ int c3d_pm_autotune(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32
     k.ntiles = pix_tiles(items.data(), (int)items.size());
     const KernelSet* ks = use_quads(s, k, run_quad8(s, k, items, 0));
     HIP_TRY(ks->eval(k, 1, st));
+    // (1, 1) stands for the default, timed with the lanes per pixel that it takes on this batch
+    const int lanes = half_lanes(items.data(), (int)items.size());
     const int cand[C3D_TILE_SHAPES][2] = {{1, 1}, {2, 1}, {4, 1}, {4, 2}};
     double ms[C3D_TILE_SHAPES] = {};
     int bestc = 0;
     for (int c = 0; c < C3D_TILE_SHAPES; ++c) {
+        const int rows = cand[c][0], tpp = c == 0 ? lanes : cand[c][1];
         KParams h = k;
         h.random_init = 0;
         ks = use_quads(s, h, run_quad8(s, k, items, 0));
-        h.ntiles = half_tiles(items.data(), (int)items.size(), cand[c][0], cand[c][1]);
-        HIP_TRY(launch_half_tile_prefix(h.batch, h.nitems, cand[c][0], cand[c][1], s->tile_pre.p, st));
+        h.ntiles = half_tiles(items.data(), (int)items.size(), rows, tpp);
+        HIP_TRY(launch_half_tile_prefix(h.batch, h.nitems, rows, tpp, s->tile_pre.p, st));
         h.tile_pre = s->tile_pre.p;
         for (int it = 0; it < 3; ++it) {
             iteration_constants(s->pm_copy, false, (uint32_t)it, h);
@@ -1723,7 +1730,7 @@ int c3d_pm_autotune(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32
             if (it == 1) HIP_TRY(hipEventRecord(s->ev[0], st));
             for (int color = 0; color < 2; ++color) {
                 h.color = color;
-                HIP_TRY(ks->half(h, cand[c][0], cand[c][1], st));
+                HIP_TRY(ks->half(h, rows, tpp, st));
             }
         }
         HIP_TRY(hipEventRecord(s->ev[1], st));
@@ -1735,7 +1742,7 @@ int c3d_pm_autotune(c3d_pm_session* s, const uint32_t* views, uint32_t n, uint32
     }
     s->half_rows = cand[bestc][0];
     s->half_tpp = cand[bestc][1];
-    s->half_auto = false;
+    s->half_below = bestc == 0 ? 0 : lanes;
     if (rows_out) *rows_out = (uint32_t)s->half_rows;
     if (tpp_out) *tpp_out = (uint32_t)s->half_tpp;
     if (ms_out)

@@ -368,9 +368,11 @@ int c3d_fill_holes_noalloc(c3d_pm_backend* backend, float* depth, float* normal,
  * shapes — (rows of pixel blocks, lanes per pixel) = (1, 1), (2, 1), (4, 1), (4, 2); 64 / lanes
  * active pixels per block — on `views` at `level` (a random initialisation and two timed
  * photometric iterations on the session's scratch states, after one untimed) and keeps the fastest
- * for the session's later runs. Every shape gives identical results. rows_out / tpp_out (optional)
- * receive the choice, ms_out[C3D_TILE_SHAPES] (optional) the times of the two iterations per shape
- * in that order. */
+ * for the session's later runs. (1, 1) stands for the default, one-wave workgroups with 1, 2, 4 or 8
+ * lanes per pixel by the pixels of each launch, and is timed as that; another choice leaves the
+ * default to launches small enough for more lanes than it takes on `views`. Every shape gives
+ * identical results. rows_out / tpp_out (optional) receive the choice, ms_out[C3D_TILE_SHAPES]
+ * (optional) the times of the two iterations per shape in that order. */
 #define C3D_TILE_SHAPES 4
 int c3d_pm_autotune(c3d_pm_session* session, const uint32_t* views, uint32_t num_views, uint32_t level,
                     uint32_t* rows_out, uint32_t* tpp_out, double* ms_out);
