@@ -1195,6 +1195,7 @@ std::vector<uint8_t> graph_key(c3d_pm_session* s, const uint32_t* views, uint32_
     put(sch, sizeof *sch);
     put(&s->half_rows, sizeof s->half_rows);
     put(&s->half_tpp, sizeof s->half_tpp);
+    put(&s->half_below, sizeof s->half_below);
     const void* ptrs[] = {s->plane.p, s->cost.p, s->bview.p, s->count.p, s->snap.p, s->plane2.p, s->need.p, s->low.p,
                           s->up.p, s->cinit.p, s->prior.p, s->d_batch_lv.p, s->d_snap_lv.p, s->tile_pre.p};
     put(ptrs, sizeof ptrs);

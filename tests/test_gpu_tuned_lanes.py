@@ -21,7 +21,8 @@ def _densify_ms(s, graph):
 
 
 @pytest.mark.parametrize("graph", [0, 1])
-def test_tuning_a_small_job_keeps_its_lanes(graph):
+@pytest.mark.parametrize("shape", [(0, 0), (1, 1)])  # untuned, and one lane asked for before tuning
+def test_tuning_a_small_job_keeps_its_lanes(graph, shape):
     sc = scenes.make_terrain_scene(scenes.oblique_rig(3), 160, 96, focal=125.0, seed=7)
     pmp, fl = abi.fast_profile()
     inp = scenes.kernel_input(sc, SRC, [(20.0, 80.0)] * 3, pmp, fl)
@@ -29,6 +30,8 @@ def test_tuning_a_small_job_keeps_its_lanes(graph):
     for tune in (0, 1):
         opts = abi.c3d_pm_options()
         opts.use_graph = graph
+        if tune:
+            opts.tile_rows, opts.threads_per_pixel = shape
         be = pm.HipPatchMatch(0, opts)
         with be.begin(inp) as s:
             if tune:
