@@ -159,6 +159,11 @@ void backend_release(c3d_pm_backend* be) {
 
 // Sessions of more quad entries (view-level pixels) keep the 4-byte table only: the second one is at most 4 GiB.
 constexpr size_t QUAD8_ENTRIES = (size_t)1 << 29;
+// So does a session on a device with less free memory than QUAD8_ROOM times the second table. Everything
+// else that a session may come to need is at most 18 times it (states, snapshot, schedule and transfers
+// 110 bytes a pixel of the top scale, post-processing 34; the table 8), so the table never takes the
+// room of a buffer that would have fitted without it.
+constexpr size_t QUAD8_ROOM = 32;
 
 struct c3d_pm_session {
     c3d_pm_backend* be = nullptr;
@@ -172,7 +177,7 @@ struct c3d_pm_session {
     // device tables
     DevBuf<uint8_t> gray;
     DevBuf<uint32_t> quad;
-    DevBuf<uint2> quad8;  // none in sessions of more than QUAD8_ENTRIES
+    DevBuf<uint2> quad8;  // see QUAD8_ENTRIES and QUAD8_ROOM
     DevBuf<LevelDesc> d_lv;
     DevBuf<PairRec> d_pairs;
     DevBuf<LevelPair> d_lpairs;
@@ -236,6 +241,15 @@ namespace {
 int set_device(c3d_pm_backend* be) {
     HIP_TRY(hipSetDevice(be->device));
     return C3D_OK;
+}
+
+// Free memory of the current device; $C3D_PM_FREE_BYTES stands in for it, so that tests can have a full one.
+size_t free_bytes() {
+    if (const char* e = std::getenv("C3D_PM_FREE_BYTES")) return (size_t)std::max(0ll, std::atoll(e));
+    size_t f = 0, total = 0;
+    if (hipMemGetInfo(&f, &total) == hipSuccess) return f;
+    (void)hipGetLastError();
+    return 0;
 }
 
 // States of `views` at `level` must match the level size (patchmatch.rs:638-642).
@@ -666,7 +680,8 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
     if (s->gray.reserve(gtot) != hipSuccess || s->quad.reserve(qtot) != hipSuccess)
         return bail(fail(C3D_DEVICE, "HIP: out of device memory for images"));
     // without room for the second table every launch takes the first
-    if (qtot <= QUAD8_ENTRIES && s->quad8.reserve(qtot) != hipSuccess) (void)hipGetLastError();
+    if (qtot <= QUAD8_ENTRIES && free_bytes() / QUAD8_ROOM >= qtot * sizeof(uint2) && s->quad8.reserve(qtot) != hipSuccess)
+        (void)hipGetLastError();
     for (int v = 0; v < nv; ++v)
         for (int l = 0; l < nl; ++l) {
             const c3d_level_image& li = in->views[v].levels[l];
