@@ -5,6 +5,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -62,8 +63,11 @@ struct c3d_init_net {
         *g_e0a;
     float *label, *range, *sums;
     float* slices = nullptr;  // partial weight gradients, from the first training step
-    float* pred = nullptr;  // c3d_init_predict's results, from its first call
-    uint8_t* img = nullptr;  // c3d_init_features' images, grown on demand
+    // workspaces of c3d_init_predict (from its first call) and c3d_init_features (grown on demand), which
+    // threads may call on one network at a time: each call holds `work` until its results are out
+    std::mutex work;
+    float* pred = nullptr;
+    uint8_t* img = nullptr;
     size_t n_img = 0;
     std::vector<float> h_range;
     std::vector<int> h_valid;  // per slot: valid width, height
@@ -418,6 +422,7 @@ int c3d_init_features(c3d_init_net* n, uint32_t slot0, uint32_t num, const c3d_s
     if (rc) return rc;
     if (!views || slot0 + num > (uint32_t)n->B) return set_error(C3D_INVALID_ARGUMENT, "slots out of range");
     hipStream_t s = n->be->stream;
+    std::lock_guard<std::mutex> g(n->work);
     // every view's images side by side in one kept buffer, so that the views' uploads and sweeps queue
     // without a wait between them
     size_t tot = 0;
@@ -584,6 +589,7 @@ int c3d_init_predict(c3d_init_net* n, uint32_t batch, float* depth, float* norma
     if (rc) return rc;
     if (batch < 1 || batch > (uint32_t)n->B) return set_error(C3D_INVALID_ARGUMENT, "batch out of range");
     hipStream_t s = n->be->stream;
+    std::lock_guard<std::mutex> g(n->work);
     rc = forward(n, (int)batch);
     if (rc) return rc;
     // the predictions are formed on the device, so that 40 bytes a pixel cross to the host at most,
