@@ -240,6 +240,58 @@ int check_net(c3d_init_net* n) {
     return C3D_OK;
 }
 
+// Device bytes of an image in c3d_init_features' buffer, and the bytes that the buffer keeps at most.
+size_t image_room(uint32_t w, uint32_t h) { return ((size_t)w * h + 255) & ~(size_t)255; }
+constexpr size_t IMG_BYTES = (size_t)64 << 20;
+
+// Uploads the images of views [a0, b0) into n->img, sweeps them and waits.
+int sweep_views(c3d_init_net* n, uint32_t slot0, const c3d_sweep_view* views, uint32_t a0, uint32_t b0) {
+    hipStream_t s = n->be->stream;
+    hipError_t e = hipSuccess;
+    size_t o = 0;
+    auto put = [&](const uint8_t* src, uint32_t w, uint32_t h) -> const uint8_t* {
+        uint8_t* dst = n->img + o;
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, (size_t)w * h, hipMemcpyHostToDevice, s);
+        o += image_room(w, h);
+        return dst;
+    };
+    for (uint32_t i = a0; i < b0 && e == hipSuccess; ++i) {
+        const c3d_sweep_view& v = views[i];
+        SweepArgs a{};
+        a.ref = put(v.gray, v.width, v.height);
+        for (uint32_t j = 0; j < v.num_sources; ++j) {
+            const c3d_sweep_source& src = v.sources[j];
+            a.src[j] = put(src.gray, src.width, src.height);
+            a.sw[j] = (int)src.width;
+            a.sh[j] = (int)src.height;
+            std::memcpy(a.sk[j], src.k, sizeof a.sk[j]);
+            std::memcpy(a.r[j], src.r, sizeof a.r[j]);
+            std::memcpy(a.t[j], src.t, sizeof a.t[j]);
+        }
+        a.rw = (int)v.width;
+        a.rh = (int)v.height;
+        std::memcpy(a.rk, v.k, sizeof a.rk);
+        a.nsrc = (int)v.num_sources;
+        a.dmin = v.depth_min;
+        a.dmax = v.depth_max;
+        a.feat = n->feat + (size_t)(slot0 + i) * n->H * n->W * 64;
+        a.H = n->H;
+        a.W = n->W;
+        if (e == hipSuccess) e = sweep(a, s);
+    }
+    // the caller's images are free again when this returns
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return set_error(C3D_DEVICE, std::string("HIP: sweep: ") + hipGetErrorString(e));
+    for (uint32_t i = a0; i < b0; ++i) {
+        n->h_range[2 * (slot0 + i)] = views[i].depth_min;
+        n->h_range[2 * (slot0 + i) + 1] = views[i].depth_max;
+        n->h_valid[2 * (slot0 + i)] = (int)views[i].width;
+        n->h_valid[2 * (slot0 + i) + 1] = (int)views[i].height;
+    }
+    return C3D_OK;
+}
+
 }  // namespace
 
 namespace c3d {
@@ -421,12 +473,10 @@ int c3d_init_features(c3d_init_net* n, uint32_t slot0, uint32_t num, const c3d_s
     int rc = check_net(n);
     if (rc) return rc;
     if (!views || slot0 + num > (uint32_t)n->B) return set_error(C3D_INVALID_ARGUMENT, "slots out of range");
-    hipStream_t s = n->be->stream;
     std::lock_guard<std::mutex> g(n->work);
-    // every view's images side by side in one kept buffer, so that the views' uploads and sweeps queue
-    // without a wait between them
-    size_t tot = 0;
-    auto room = [](uint32_t w, uint32_t h) { return ((size_t)w * h + 255) & ~(size_t)255; };
+    // images of several views side by side in one kept buffer, up to IMG_BYTES of them or those of one
+    // view, so that the views' uploads and sweeps queue without a wait between them
+    std::vector<size_t> sizes;
     uint32_t good = 0;  // views before the first bad one: they are done, as if each had its own call
     int bad = C3D_OK;
     for (; good < num; ++good) {
@@ -439,60 +489,26 @@ int c3d_init_features(c3d_init_net* n, uint32_t slot0, uint32_t num, const c3d_s
             bad = set_error(C3D_INVALID_ARGUMENT, "bad depth range");
             break;
         }
-        tot += room(v.width, v.height);
-        for (uint32_t j = 0; j < v.num_sources; ++j) tot += room(v.sources[j].width, v.sources[j].height);
+        size_t tot = image_room(v.width, v.height);
+        for (uint32_t j = 0; j < v.num_sources; ++j) tot += image_room(v.sources[j].width, v.sources[j].height);
+        sizes.push_back(tot);
     }
-    if (tot > n->n_img) {
-        if (n->img) {
-            NN_TRY(hipStreamSynchronize(s));
-            (void)hipFree(n->img);
-        }
+    auto drop = [&] {  // nothing queued reads the buffer
+        if (n->img) (void)hipFree(n->img);
         n->img = nullptr;
         n->n_img = 0;
-        NN_TRY(hipMalloc((void**)&n->img, tot));
-        n->n_img = tot;
-    }
-    hipError_t e = hipSuccess;
-    size_t o = 0;
-    auto put = [&](const uint8_t* src, uint32_t w, uint32_t h) -> const uint8_t* {
-        uint8_t* dst = n->img + o;
-        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, (size_t)w * h, hipMemcpyHostToDevice, s);
-        o += room(w, h);
-        return dst;
     };
-    for (uint32_t i = 0; i < good && e == hipSuccess; ++i) {
-        const c3d_sweep_view& v = views[i];
-        SweepArgs a{};
-        a.ref = put(v.gray, v.width, v.height);
-        for (uint32_t j = 0; j < v.num_sources; ++j) {
-            const c3d_sweep_source& src = v.sources[j];
-            a.src[j] = put(src.gray, src.width, src.height);
-            a.sw[j] = (int)src.width;
-            a.sh[j] = (int)src.height;
-            std::memcpy(a.sk[j], src.k, sizeof a.sk[j]);
-            std::memcpy(a.r[j], src.r, sizeof a.r[j]);
-            std::memcpy(a.t[j], src.t, sizeof a.t[j]);
+    for (uint32_t a = 0, b; a < good; a = b) {
+        size_t tot = sizes[a];
+        for (b = a + 1; b < good && tot + sizes[b] <= IMG_BYTES; ++b) tot += sizes[b];
+        if (tot > n->n_img) {
+            drop();
+            NN_TRY(hipMalloc((void**)&n->img, tot));
+            n->n_img = tot;
         }
-        a.rw = (int)v.width;
-        a.rh = (int)v.height;
-        std::memcpy(a.rk, v.k, sizeof a.rk);
-        a.nsrc = (int)v.num_sources;
-        a.dmin = v.depth_min;
-        a.dmax = v.depth_max;
-        a.feat = n->feat + (size_t)(slot0 + i) * n->H * n->W * 64;
-        a.H = n->H;
-        a.W = n->W;
-        if (e == hipSuccess) e = sweep(a, s);
-    }
-    // the caller's images are free again when this returns
-    const hipError_t es = hipStreamSynchronize(s);
-    if (e == hipSuccess) e = es;
-    if (e != hipSuccess) return set_error(C3D_DEVICE, std::string("HIP: sweep: ") + hipGetErrorString(e));
-    for (uint32_t i = 0; i < good; ++i) {
-        n->h_range[2 * (slot0 + i)] = views[i].depth_min;
-        n->h_range[2 * (slot0 + i) + 1] = views[i].depth_max;
-        n->h_valid[2 * (slot0 + i)] = (int)views[i].width;
-        n->h_valid[2 * (slot0 + i) + 1] = (int)views[i].height;
+        rc = sweep_views(n, slot0, views, a, b);
+        if (n->n_img > IMG_BYTES) drop();
+        if (rc) return rc;
     }
     return bad;
 }
