@@ -529,6 +529,12 @@ __device__ __forceinline__ bool homography(const LevelDesc& R, const LevelPair& 
 // one mixed FMA on them: the same value as the FP32 formula. From a 4-byte entry p00 | p10 << 8 |
 // p01 << 16 | p11 << 24 they take a byte permute each that sets the exponent byte 0x64 above each
 // texel, which reads 1024 + p exactly, and a packed subtraction each; an 8-byte entry holds them.
+// Everything from here on is compiled once per entry size, and so has a namespace per entry size.
+#if C3D_QUAD_BYTES == 8
+inline namespace entry8 {
+#else
+inline namespace entry4 {
+#endif
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t quad_entry4(uint32_t p00, uint32_t p10, uint32_t p01, uint32_t p11) {
     return p00 | (p10 << 8) | (p01 << 16) | (p11 << 24);
@@ -1112,4 +1118,5 @@ __device__ __forceinline__ float4 eval_init_plane(const KParams& P, const ViewDe
     return h;
 }
 
+}  // namespace entry4 / entry8
 }  // namespace c3d
