@@ -108,7 +108,10 @@ struct KParams {
 // in that L2, and the runs are dealt to the XCDs in turn, so that every XCD gets its share of the
 // costly and of the cheap parts of each view. (One contiguous eighth of the tiles per XCD left
 // XCDs idle while the one with the costliest eighth finished: 1.7 of 2 wave slots per SIMD were
-// taken on average.) In the half step a run is a square of 8 x 8 blocks (HALF_BAND), 128 x 64 pixels.
+// taken on average.) In the half step a run is a square of 8 x 8 blocks (HALF_BAND), 128 x 64 pixels,
+// with one-row workgroups; with 2 and 4 rows a run's 64 workgroups are 8 blocks high and 16 and 32 wide.
+// The kernels of 64 x 4 and 128 x 4 pixel tiles (evaluation, read-out, upsampling, median) take runs of
+// 64 tiles row by row; runs were compared on the half step only.
 // Each round of 8 runs starts at another XCD, scattered by a multiplicative hash: without it a width
 // of a whole or half number of rounds gives each XCD the same columns of every view. Measured against
 // runs of 16 tiles of one row: half step of 9 views of 1920 x 1080 with 6 sources 17.91 -> 17.72 ms; 2
@@ -188,7 +191,9 @@ __device__ __forceinline__ bool find_tile(const KParams& P, int t, int tw, int t
 // 4), picked per session by the tile autotuner (c3d_pm_autotune). One is the default: a wave's slot
 // on its SIMD is refilled as soon as that wave ends, where a 4-wave workgroup holds its slots (and
 // its LDS) until its slowest wave is done, and the waves' work differs through the data-dependent
-// early exits.
+// early exits. On the other hand 4-wave workgroups take less LDS a wave (the margins of the staged
+// pixels are shared; a one-wave workgroup holds 12,096 bytes and 256 a source). Jobs from random
+// planes are often faster with them, which is what the tuner is for.
 constexpr int HALF_SPAN = 128;   // pixel span of one row of 64 active pixels (k_eval of one colour)
 // A wave of the half step takes a block of half_bw x half_bh pixels, half of them active: 16 x 8, or
 // 8 x 8, 8 x 4 and 8 x 2 with two, four and eight lanes per pixel. What

@@ -356,10 +356,9 @@ KParams params_for(c3d_pm_session* s, uint32_t level, bool geometric, const std:
     return k;
 }
 
-// The top-scale results of a densify call copied straight into the caller's arrays: the planes
-// are split into depth and 3-float normal arrays on the device, then each view's depth, normal,
-// cost, raw depth and count come back with one transfer each, in stream order, and one final
-// synchronisation (no host staging buffer, no host-side unpacking).
+// The top-scale results of a densify call copied into the caller's arrays: the planes are split into
+// depth and 3-float normal arrays on the device, then each view's depth, normal, cost, raw depth and
+// count come back through the staging buffers (c3d::download), with no host-side unpacking.
 int download_results(c3d_pm_session* s, const BatchItem* items, uint32_t n, long long npix, c3d_view_state* out,
                      uint8_t* const* counts, float* const* raw_depth);
 int download_states(c3d_pm_session* s, const float4* plane, const float* cost, const BatchItem* items, uint32_t n, long long npix,
@@ -631,7 +630,8 @@ int c3d_pm_begin(c3d_pm_backend* be, const c3d_kernel_input* in, c3d_pm_session*
         for (int l = 0; l < nl; ++l) {
             if (!kv.levels[l].gray || kv.levels[l].width < 1 || kv.levels[l].height < 1)
                 return fail(C3D_INVALID_ARGUMENT, "empty level image");
-            // source-sample table byte offsets are formed exactly in FP32 (multiples of 4 below 2^26)
+            // source-sample table byte offsets are formed exactly in FP32 (multiples of 4 below 2^26, or of 8
+            // below 2^27)
             if (((uint64_t)kv.levels[l].width + 3) * ((uint64_t)kv.levels[l].height + 3) > (1ULL << 24))
                 return fail(C3D_INVALID_ARGUMENT, "image larger than (w + 3)(h + 3) <= 2^24 pixels");
         }

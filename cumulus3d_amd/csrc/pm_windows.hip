@@ -25,8 +25,9 @@ namespace c3d {
 namespace C3D_QUAD_NS {
 
 // The run-start evaluation and the read-out keep five source gathers in flight through a window
-// and, for register-held windows of at most 36 samples, ask for three waves per SIMD: 156-158
-// VGPRs without spills (eight in flight needed 180-187 VGPRs, two waves per SIMD).
+// and, for register-held windows of at most 36 samples, ask for three waves per SIMD: 117-141
+// VGPRs for the (5, 2) window, no spills. (The depth was chosen on an earlier window loop, which took
+// 156-158 VGPRs with five and 180-187, two waves per SIMD, with eight.)
 constexpr int EVAL_PIPE = 5;
 template <int WR, int WSTEP>
 constexpr int eval_waves() {
@@ -110,9 +111,9 @@ __global__ __launch_bounds__(ROWS * 64) __attribute__((amdgpu_waves_per_eu(half_
 void k_half(KParams P) {
     constexpr int NT = ROWS * 64;
     constexpr int BW = half_bw(TPP), BH = half_bh(TPP) * ROWS;  // pixels of the workgroup's block
-    // source gathers in flight in the window loop: four for three waves per SIMD (166 VGPRs
-    // photometric; deeper spills and measures no faster), six for two waves, fewer for the 49
-    // register-held weights of a 7 x 7 window
+    // source gathers in flight in the window loop: four for three waves per SIMD (the 168 VGPRs of
+    // that and two spilled, 12 bytes of scratch a lane; deeper spills more and measures no faster),
+    // six for two waves (221-237 VGPRs), fewer for the 49 register-held weights of a 7 x 7 window
     constexpr int PIPE = Win<(WR > 0 ? WR : 1), WSTEP>::WN2 > 36 ? 3 : (FEW ? 6 : 4);
     // the reference value of a window sample is read with its gather (see window_sums)
     constexpr bool AHEAD = Win<(WR > 0 ? WR : 1), WSTEP>::WN2 <= 36;
