@@ -63,9 +63,10 @@ HBM_PEAK_GBS = 8000.0
 # Keyed by workload and the half step's workgroup shape (rows, lanes per pixel), which changes the
 # fetched bytes; other shapes report null:
 #   zone7, (1, 1): 7 x 1920x1080, 6 sources, 7 + 1x2 iterations, averaged over its 18 launches
+#          (profiles/k_half-zone7-7x1080p-6src.md)
 #   zone108_1_1x1, (1, 1): the 108-view zone's learned job, 1 refinement + 1x1 geometric
 #          iterations, averaged over its 4 launches (profiles/k_half-zone108-learned.md)
-K_HALF_TRAFFIC = {("zone7", (1, 1)): 12.035e9, ("zone108_1_1x1", (1, 1)): 176.289e9}
+K_HALF_TRAFFIC = {("zone7", (1, 1)): 12.110e9, ("zone108_1_1x1", (1, 1)): 176.151e9}
 FP32_PEAK_TFLOPS = 157.3
 FLOP_PER_SAMPLE = 28  # projective transform 9, reciprocal 1, bilinear 7, scale 1, accumulations 6 (rounded up)
 WN_FAST = 6  # samples per window side at radius 5 step 2

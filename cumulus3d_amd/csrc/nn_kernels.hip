@@ -657,9 +657,9 @@ hipError_t sweep(const SweepArgs& a, hipStream_t s) {
 // ---------------------------------------------------------------- network output -> predictions
 //
 // Bound by the transfer to the host. With the predictions formed on the host from the padded 128-byte
-// head output of each pixel, features and prediction of 6 images of 480 x 272 took 13.9 ms; formed
-// here, 40 bytes a pixel cross at most, and both take 2.7 ms together (the convolutions' share of the
-// gain is 0.9).
+// head output of each pixel, features and prediction of 6 images of 480 x 272 took 13.9 to 32.8 ms, by
+// process (a host vector of 100 MB a call); formed here, 40 bytes a pixel cross at most, and both take
+// 2.7 to 3.7 ms together (the convolutions' share of the gain is 0.9).
 
 __global__ __launch_bounds__(256) void k_predict(PredictArgs a) {
     const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
